@@ -108,6 +108,7 @@ struct Layout {
   cgdev::GeomT<R> g{};
   int ncv = 0, nfa = 0, nef = 0, nblocks = 0, npblocks = 0;
   size_t lds = 0;             // LDS bytes of its extended-face halo (0: no halo)
+  size_t slds = 0;            // the same of its slices' halos (0: none)
   int* solo_bmap = nullptr;   // cell blocks in XCD order
   int* solo_pbmap = nullptr;  // compact-pair blocks in XCD order
   // device cell i holds mesh cell ext_of[i]: every 256-cell block keeps its
@@ -180,7 +181,7 @@ struct Instance : HostInst {
   cgdev::Inst<R>* solo = nullptr;    // one-entry device table of this instance
   int slot = -1;                     // its entry in its engine's device table
   cgk::Launch<R> solo_launch() const {
-    return {solo, lay->solo_bmap, nblocks, 1, lds, lay->solo_pbmap, npblocks, 4, prm.sgs_model == CG_SGS_SIGMA,
+    return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, 4, prm.sgs_model == CG_SGS_SIGMA,
             prm.use_full_gr != 0, prm.sgs_model == CG_SGS_DSM_LOCAL, prm.nsc,
             scalar_lds<R>(lds, prm.nsc, lay->lds_max), lay->g.nbf > 0, zsum, wm ? lay->g.nbf : 0};
   }
@@ -738,13 +739,18 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
       const int nblk = (ncv + cgdev::kBlock - 1) / cgdev::kBlock;
       std::vector<std::vector<int>> halos(nblk);
       std::vector<int16_t> loc(xs.nslots, 0);
+      // slices' halos: the subsets of their block's that each slice reaches
+      const bool slices = nblk <= cgk::kRowsMaxBlocks;
+      const int nsl = slices ? (ncv + cgdev::kSlice - 1) / cgdev::kSlice : 0;
+      std::vector<std::vector<int>> shalos(nsl);
+      std::vector<int16_t> sloc(slices ? xs.nslots : 0, 0);
       std::string herr;
       std::mutex hmu;
       const int nth = cgmesh::default_threads();
       std::vector<std::thread> th;
       for (int t = 0; t < nth; ++t)
         th.emplace_back([&, t] {
-          std::vector<int> v;
+          std::vector<int> v, to;
           for (int bk = t; bk < nblk; bk += nth) {
             // lane positions q0..q1 of the block hold the block's own cells q0..q1
             const int q0 = bk * cgdev::kBlock, q1 = std::min(ncv, q0 + cgdev::kBlock);
@@ -767,6 +773,23 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
                 const int pos = int(std::lower_bound(v.begin(), v.end(), nb) - v.begin());
                 loc[sidx] = int16_t(pos | ((xnbr[sidx] < 0) ? 0x8000 : 0));
               }
+            for (int q2 = q0; slices && q2 < q1; q2 += cgdev::kSlice) {
+              const int q3 = std::min(q1, q2 + cgdev::kSlice);
+              to.assign(v.size(), -1);
+              for (int q = q2; q < q3; ++q)
+                for (int k = 0; k < xcnt[q]; ++k) to[loc[xs.slot(q, k)] & 0x7fff] = 0;
+              std::vector<int>& sv = shalos[q2 / cgdev::kSlice];
+              for (size_t i = 0; i < v.size(); ++i)
+                if (to[i] == 0) {
+                  to[i] = int(sv.size());
+                  sv.push_back(v[i]);
+                }
+              for (int q = q2; q < q3; ++q)
+                for (int k = 0; k < xcnt[q]; ++k) {
+                  const int64_t sidx = xs.slot(q, k);
+                  sloc[sidx] = int16_t(to[loc[sidx] & 0x7fff] | (loc[sidx] & 0x8000));
+                }
+            }
             halos[bk] = v;
           }
         });
@@ -791,6 +814,21 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
         rc |= upload(s, h, &g.xf_loc, loc);
         g.halo_max = hmax;
         Lay->lds = (size_t)hmax * 6 * sizeof(R);
+        if (slices) {
+          std::vector<int> sptr(nsl + 1, 0), sv;
+          size_t smax = 1;
+          for (int i = 0; i < nsl; ++i) {
+            sv.insert(sv.end(), shalos[i].begin(), shalos[i].end());
+            sptr[i + 1] = int(sv.size());
+            smax = std::max(smax, shalos[i].size());
+          }
+          rc |= upload(s, h, &g.sh_ptr, sptr);
+          rc |= upload(s, h, &g.sh_v, sv);
+          rc |= upload(s, h, &g.sh_loc, sloc);
+          // beside the pass's static 105 rows of 64 values
+          const size_t sb = smax * 6 * sizeof(R);
+          if (sb + 105 * cgdev::kSlice * sizeof(R) <= (size_t)lds_max) Lay->slds = sb;
+        }
       }
     }
     rc |= upload(s, h, &g.cf_ptr, cs.ptr);
@@ -998,6 +1036,7 @@ int build_instance(Err* s, Instance<R>* I, std::shared_ptr<Layout<R>> lay, const
   rc |= dev_alloc(s, h, &w.rhs0, 5 * (size_t)ncv);
   rc |= dev_alloc(s, h, &w.rhs1, 5 * (size_t)ncv);
   rc |= dev_alloc(s, h, &w.cflux, 6 * (size_t)std::max(nfa, 1));
+  if (lay->g.nbf > 0) rc |= dev_alloc(s, h, &w.bacc, 5 * (size_t)ncv);
   rc |= dev_alloc(s, h, &hi->info, 1);
   w.info = hi->info;
   rc |= dev_alloc(s, h, &w.partial, 8 * (size_t)hi->nblocks);
@@ -1133,8 +1172,8 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
   const int n = (int)E.inst.size();
   std::vector<cgdev::Inst<R>> tab(n);
   std::vector<int> logical, plogical;  // logical block -> (instance, local block)
-  size_t lds = 0;
-  bool all_halo = true;
+  size_t lds = 0, slds = 0;
+  bool all_halo = true, all_shalo = true;
   for (int i = 0; i < n; ++i) {
     Instance<R>* I = E.inst[i];
     tab[i] = I->record();
@@ -1143,6 +1182,8 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
     for (int b = 0; b < I->npblocks; ++b) plogical.push_back((i << cgdev::kBlkBits) | b);
     lds = std::max(lds, I->lds);
     all_halo = all_halo && I->lds > 0;
+    slds = std::max(slds, I->lay->slds);
+    all_shalo = all_shalo && I->lay->slds > 0;
   }
   auto ordered = [](const std::vector<int>& lg) {
     std::vector<int> out(lg.size());
@@ -1192,7 +1233,7 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
   E.h_pbmap = pbmap;
   E.hole_blocks = 0;
   const size_t flux_lds = (all_halo && !E.force_global) ? lds : 0;
-  E.L = {E.tab, E.bmap, nb, n, flux_lds, E.pbmap, npb, E.tile, any_sigma,
+  E.L = {E.tab, E.bmap, nb, n, flux_lds, flux_lds && all_shalo ? slds : 0, E.pbmap, npb, E.tile, any_sigma,
          any_full_gr, any_dsm, max_nsc, scalar_lds<R>(flux_lds, max_nsc, lds_max), any_bf, any_zsum,
          wm_nbf};
   E.dirty = false;

@@ -85,6 +85,10 @@ struct GeomT {
   const int *halo_ptr, *halo_v;
   const int16_t* xf_loc;
   int halo_max;
+  // the same per 64-cell slice (null on meshes too large for the row-split
+  // passes): sh_v[sh_ptr[s] .. sh_ptr[s+1]), sh_loc as xf_loc
+  const int *sh_ptr, *sh_v;
+  const int16_t* sh_loc;
   // gradient stencil without the diagonal, SELL-64 layout in its own lane
   // order (gperm, as xperm)
   const uint8_t* gperm;
@@ -129,6 +133,7 @@ struct WorkT {
   R* rhs0;           // [5][ncv]
   R* rhs1;           // [5][ncv]
   R* cflux;          // [nfa][6] flux of each compact pair (lo -> hi), this stage
+  R* bacc;           // [5][ncv] boundary part of the boundary cells' RHS (null without boundary faces)
   StepInfo* info;
   double* partial;   // reduction scratch [nblocks][8]
   double* diag;      // [8]
@@ -242,6 +247,9 @@ constexpr int kBlkBits = 20;  // up to 2^20 blocks (268M cells) per instance, 2^
 // launches, `lds` the dynamic LDS bytes of the extended-face pass (0: the
 // global-gather variant; every instance then needs no halo).
 namespace cgk {
+// the most cell blocks of a launch that takes the row-split passes: layouts of
+// larger meshes carry no slice halos
+constexpr int kRowsMaxBlocks = 384;
 template <class R>
 struct Launch {
   const cgdev::Inst<R>* I;
@@ -249,6 +257,7 @@ struct Launch {
   int nblk;
   int ninst;
   size_t lds;
+  size_t slds;       // dynamic LDS bytes of the row-split flux pass (0: not available)
   const int* pbmap;  // compact-pair blocks
   int npblk;
   int tile;          // extended slots fetched per batch in the LDS pass (2, 4 or 8)

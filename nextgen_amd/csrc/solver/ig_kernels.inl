@@ -224,7 +224,7 @@ __device__ __forceinline__ float flip(float x, bool neg) {
 }
 
 // One extended half-face's pair flux (skew + symmetric, in the pair's lo -> hi
-// orientation) added to the cell's accumulation: -F on the lo side, +F on the
+// orientation) signed for the cell's accumulation: -F on the lo side, +F on the
 // hi side. Evaluated from the cell's own side, (self, other), with no select
 // of the two records: every operation of flux_skew is symmetric in its two
 // states (sums, products, averages), so its result is the same bits for
@@ -235,9 +235,9 @@ __device__ __forceinline__ float flip(float x, bool neg) {
 //   F(lo, hi) = skew(self, other) + (self is hi ? -1 : 1) symmetric(self, other)
 // bit for bit, and acc - F == acc + (-F).
 template <class R>
-__device__ __forceinline__ void add_half_face(R acc[5], const R n[3], const R cv[3], const Light<R>& self,
-                                              const Light<R>& other, bool self_hi) {
-  R F[5], u_avg[3], inv_v_avg, h_stag;
+__device__ __forceinline__ void half_face_flux(R F[5], const R n[3], const R cv[3], const Light<R>& self,
+                                               const Light<R>& other, bool self_hi) {
+  R u_avg[3], inv_v_avg, h_stag;
   flux_skew(F, n, self, other, u_avg, inv_v_avg, h_stag);
   if (cv[0] != R(0) || cv[1] != R(0) || cv[2] != R(0)) {
     R cF[5];
@@ -246,7 +246,16 @@ __device__ __forceinline__ void add_half_face(R acc[5], const R n[3], const R cv
     for (int q = 0; q < 5; ++q) F[q] += flip(cF[q], self_hi);
   }
 #pragma unroll
-  for (int q = 0; q < 5; ++q) acc[q] += flip(F[q], !self_hi);
+  for (int q = 0; q < 5; ++q) F[q] = flip(F[q], !self_hi);
+}
+
+template <class R>
+__device__ __forceinline__ void add_half_face(R acc[5], const R n[3], const R cv[3], const Light<R>& self,
+                                              const Light<R>& other, bool self_hi) {
+  R F[5];
+  half_face_flux(F, n, cv, self, other, self_hi);
+#pragma unroll
+  for (int q = 0; q < 5; ++q) acc[q] += F[q];
 }
 
 // calcInternalCompactFluxNewGrad, IdealGasSolverFlux.hpp:93-215. In mixed
@@ -1185,6 +1194,21 @@ __device__ __forceinline__ R boundary_cfl(const GeomT<R>& g, int c, const Light<
   return cfl;
 }
 
+// whether the boundary part of cell c's RHS is not identically zero
+template <class R>
+__device__ __forceinline__ bool has_boundary(const GeomT<R>& g, const Params& P, int c) {
+  return P.sponge_zone >= 0 || G(g.bf_ptr)[c + 1] > G(g.bf_ptr)[c];
+}
+
+// the boundary part of cell c's RHS, as k_bflux left it
+template <class R>
+__device__ __forceinline__ void boundary_part(const GeomT<R>& g, const WorkT<R>& w, const Params& P, int c,
+                                              R acc[5]) {
+  const bool has = g.nbf > 0 && has_boundary(g, P, c);
+#pragma unroll
+  for (int q = 0; q < 5; ++q) acc[q] = has ? R(G(w.bacc)[(size_t)q * g.ncv + c]) : R(0);
+}
+
 // The compact-pair fluxes, in pair order, of the cell at lane position pos
 // (its first ef_nc pairs), added to its stage RHS accumulation.
 template <class R>
@@ -1338,6 +1362,329 @@ __global__ __launch_bounds__(kBlock) void k_flux_lds(const Inst<R>* __restrict__
     return;
   }
   rk_update<STAGE>(g, in, out, w, P, c, self, acc);
+}
+
+// x as it stands: keeps a load ahead of the select that uses it, which the
+// compiler would otherwise turn into a branch around the load
+template <class T>
+__device__ __forceinline__ T pinned(T x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// Boundary part of a stage for the passes that do not carry it: the faces' (and
+// a sponge's) contributions to each boundary cell's RHS into w.bacc[5][ncv],
+// with the faces' own stage updates. Thread per cell. Kept out of those passes
+// because its ~100 registers would halve their wavefronts.
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_bflux(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
+                                                  int cur, int stage, int update) {
+  int lblk;
+  const Inst<R>* Xp = inst_of(I, bmap, lblk);
+  if (!Xp) return;
+  const Inst<R>& X = *Xp;
+  const GeomT<R> g = X.g;
+  const WorkT<R> w = X.w;
+  const int c = lblk * kBlock + threadIdx.x;
+  if (c >= g.ncv || g.nbf == 0) return;
+  if (update && G(w.info)->nan) return;
+  if (!has_boundary(g, X.P, c)) return;
+  const StateT<R> in = X.st[cur];
+  R acc[5];
+  boundary_flux(g, w, in, X.P, c, load_light(in.light, c), acc, stage, update != 0);
+#pragma unroll
+  for (int q = 0; q < 5; ++q) G(w.bacc)[(size_t)q * g.ncv + c] = acc[q];
+}
+
+// The thread-per-cell LDS pass with its loads pipelined, for launches of a few
+// workgroups per CU: rows are fetched kNB at a time, the next kNB while these are
+// added. No load is under a branch, so that the wait for one batch leaves the
+// next in flight: a lane past its last row (and every lane past the slice's
+// last) reads its slice's first slot of the row, a line that is fetched anyway,
+// and its flux is not added. The accumulation order stays k = 0, 1, ...
+template <class R, int STAGE, int MODE>
+__global__ __launch_bounds__(kBlock) void k_flux_pipe(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
+                                                      int cur, double* rhs_out) {
+  using T2 = typename V2<R>::T;
+  constexpr int kNB = 2;  // extended rows per batch
+  constexpr int kC = 4;   // compact rows per batch
+  extern __shared__ __align__(16) unsigned char smem[];
+  T2* halo = reinterpret_cast<T2*>(smem);  // [hsize][3]
+  int blk;
+  const Inst<R>* Xp = inst_of(I, bmap, blk);
+  if (!Xp) return;
+  const Inst<R>& X = *Xp;
+  const GeomT<R> g = X.g;
+  const StateT<R> in = X.st[cur], out = X.st[cur ^ 1];
+  const WorkT<R> w = X.w;
+  const Params& P = X.P;
+  if (MODE == 1 && G(w.info)->nan) return;
+  const int hb = G(g.halo_ptr)[blk], hs = G(g.halo_ptr)[blk + 1] - hb;
+  for (int i = threadIdx.x; i < hs; i += kBlock) {
+    const auto q = G(in.light + (size_t)G(g.halo_v)[hb + i] * L_N);
+    halo[3 * i + 0] = mk2(q[0], q[1]);
+    halo[3 * i + 1] = mk2(q[2], q[3]);
+    halo[3 * i + 2] = mk2(q[4], q[5]);
+  }
+  __syncthreads();
+  const int pos0 = blk * kBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice) * kSlice;
+  const int lane = threadIdx.x & (kSlice - 1), pos = pos0 + lane;
+  if (pos >= g.ncv) return;
+  const int c = cell_at(g.xperm, pos);
+  const int sl = pos0 / kSlice;
+  const int xp0 = G(g.xf_ptr)[sl], nrow = (G(g.xf_ptr)[sl + 1] - xp0) / kSlice;
+  const int cp0 = G(g.cf_ptr)[sl], ncrow = (G(g.cf_ptr)[sl + 1] - cp0) / kSlice;
+  const int deg = G(g.xf_deg)[pos], nc = G(g.ef_nc)[pos];
+  const int ncv = g.ncv;
+  const Light<R> self = load_light(in.light, c);
+  R acc[5];
+  boundary_part(g, w, P, c, acc);
+  if (ncrow > 0) {
+    int code[kC];
+    auto ld = [&](int k0) {
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        const int k = k0 + j;
+        code[j] = ldnt(g.cf_pair + cp0 + (k < ncrow ? k : ncrow - 1) * kSlice + (k < nc ? lane : 0));
+      }
+    };
+    ld(0);
+    for (int k0 = 0; k0 < ncrow; k0 += kC) {
+      R F[kC][5];
+      bool neg[kC];
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        const int f = k0 + j < nc ? pinned(code[j]) & 0x7fffffff : 0;
+        neg[j] = code[j] >= 0;
+        const auto fl = G(w.cflux + (size_t)f * 6);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) F[j][q] = fl[q];
+      }
+      ld(k0 + kC);
+#pragma unroll
+      for (int j = 0; j < kC; ++j)
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+          const R sum = acc[q] + flip(pinned(F[j][q]), neg[j]);
+          acc[q] = k0 + j < nc ? sum : acc[q];
+        }
+    }
+  }
+  struct Row {
+    R n[3], cv[3];
+    int code;
+  };
+  auto ld = [&](Row(&r)[kNB], int k0) {
+#pragma unroll
+    for (int j = 0; j < kNB; ++j) {
+      const int k = k0 + j;
+      const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < deg ? lane : 0);
+      r[j].code = ldnt(g.xf_loc + slot);
+      r[j].n[0] = ldnt(g.xsn0 + slot); r[j].n[1] = ldnt(g.xsn1 + slot); r[j].n[2] = ldnt(g.xsn2 + slot);
+      r[j].cv[0] = ldnt(g.xsc0 + slot); r[j].cv[1] = ldnt(g.xsc1 + slot); r[j].cv[2] = ldnt(g.xsc2 + slot);
+    }
+  };
+  auto add = [&](const Row(&r)[kNB], int k0) {
+#pragma unroll
+    for (int j = 0; j < kNB; ++j) {
+      const int li = r[j].code & 0x7fff;
+      const T2 r0 = halo[3 * li + 0], r1 = halo[3 * li + 1], r2 = halo[3 * li + 2];
+      Light<R> other;
+      other.u[0] = r0.x; other.u[1] = r0.y; other.u[2] = r1.x; other.spv = r1.y; other.p = r2.x; other.h = r2.y;
+      other.rho = R(0); other.sos = R(0);
+      R F[5];
+      half_face_flux(F, r[j].n, r[j].cv, self, other, (r[j].code & 0x8000) != 0);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        const R sum = acc[q] + F[q];
+        acc[q] = k0 + j < deg ? sum : acc[q];
+      }
+    }
+  };
+  if (nrow > 0) {
+    Row ra[kNB], rb[kNB];
+    ld(ra, 0);
+    int k0 = 0;
+    for (; k0 + 2 * kNB < nrow; k0 += 2 * kNB) {
+      ld(rb, k0 + kNB);
+      add(ra, k0);
+      ld(ra, k0 + 2 * kNB);
+      add(rb, k0 + kNB);
+    }
+    if (k0 + kNB < nrow) ld(rb, k0 + kNB);
+    add(ra, k0);
+    if (k0 + kNB < nrow) add(rb, k0 + kNB);
+  }
+  if (MODE == 0) {
+    write_rhs(rhs_out, ncv, c, acc, P);
+    return;
+  }
+  rk_update<STAGE>(g, in, out, w, P, c, self, acc);
+}
+
+// Slice of this workgroup when each cell block is split in its kBlock / kSlice
+// slices, one per workgroup: the slices of a block keep its XCD (consecutive
+// workgroups are dealt round-robin over the XCDs). The grid has slice_grid(nblk)
+// workgroups; null beyond the block map and for its empty entries.
+constexpr int kSlicesPerBlock = kBlock / kSlice;
+inline int slice_grid(int nblk) { return (nblk + kXcd - 1) / kXcd * kXcd * kSlicesPerBlock; }
+template <class R>
+__device__ __forceinline__ const Inst<R>* slice_of(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
+                                                   int nblk, int& pos0) {
+  const int x = blockIdx.x % kXcd, j = blockIdx.x / kXcd;
+  const int b = (j / kSlicesPerBlock) * kXcd + x;
+  if (b >= nblk) return nullptr;
+  const int e = bmap[b];
+  if (e < 0) return nullptr;
+  pos0 = (e & ((1 << kBlkBits) - 1)) * kBlock + (j % kSlicesPerBlock) * kSlice;
+  const Inst<R>* X = I + (e >> kBlkBits);
+  return pos0 < X->g.ncv ? X : nullptr;
+}
+
+// Barrier of a workgroup that exchanges values through LDS only: global loads
+// in flight stay in flight across it (__syncthreads would wait for them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The extended-face pass split by rows, for launches too small to fill the chip
+// with a thread per cell (a wavefront then walks its ~65 half-faces in a row,
+// bound by the latency of their loads). One workgroup of W wavefronts
+// takes one slice: it stages the records its extended half-faces reach (the
+// slice's halo) in LDS, wavefront w evaluates the pair fluxes of rows w, w + W,
+// ... of the slice's SELL regions (a row is one half-face of each of the 64
+// cells) into LDS, and after each group of W rows wavefront q < 5 adds the group's
+// rows, in order, to component q of its 64 cells. Every sum keeps the order of
+// the thread-per-cell pass, so both give the same bits.
+template <class R, int STAGE, int MODE, int W>
+__global__ __launch_bounds__(W* kSlice) void k_flux_rows(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
+                                                         int nblk, int cur, double* rhs_out) {
+  using T2 = typename V2<R>::T;
+  constexpr int kC = 20 / W;  // compact rows per wavefront requested together (even: box alternates)
+  extern __shared__ __align__(16) unsigned char smem[];
+  T2* halo = reinterpret_cast<T2*>(smem);  // [hsize][3]
+  __shared__ R box[2][W][5][kSlice];
+  __shared__ R fin[5][kSlice];
+  int pos0 = 0;
+  const Inst<R>* Xp = slice_of(I, bmap, nblk, pos0);
+  if (!Xp) return;
+  const Inst<R>& X = *Xp;
+  const GeomT<R> g = X.g;
+  const StateT<R> in = X.st[cur], out = X.st[cur ^ 1];
+  const WorkT<R> w = X.w;
+  const Params& P = X.P;
+  if (MODE == 1 && G(w.info)->nan) return;
+  const int lane = threadIdx.x & (kSlice - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice);
+  const int pos = pos0 + lane;
+  const bool live = pos < g.ncv;
+  const int c = live ? cell_at(g.xperm, pos) : pos0;
+  const int sl = pos0 / kSlice;
+  const int xp0 = G(g.xf_ptr)[sl], nrow = (G(g.xf_ptr)[sl + 1] - xp0) / kSlice;
+  const int cp0 = G(g.cf_ptr)[sl], ncrow = (G(g.cf_ptr)[sl + 1] - cp0) / kSlice;
+  const int deg = live ? G(g.xf_deg)[pos] : 0, nc = live ? G(g.ef_nc)[pos] : 0;
+  const int ncv = g.ncv;
+  const int hb = G(g.sh_ptr)[sl], hs = G(g.sh_ptr)[sl + 1] - hb;
+  // A row's neighbour code and geometry. No load is under a branch, so later
+  // rows' loads stay in flight while earlier ones are used: a lane past its last
+  // row (and every lane past the slice's last) reads lane 0's slot, a line that
+  // is fetched anyway, and its flux is not added.
+  struct Row {
+    R n[3], cv[3];
+    int code;
+  };
+  auto ld_row = [&](Row& r, int k) {
+    const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < deg ? lane : 0);
+    r.code = ldnt(g.sh_loc + slot);
+    r.n[0] = ldnt(g.xsn0 + slot); r.n[1] = ldnt(g.xsn1 + slot); r.n[2] = ldnt(g.xsn2 + slot);
+    r.cv[0] = ldnt(g.xsc0 + slot); r.cv[1] = ldnt(g.xsc1 + slot); r.cv[2] = ldnt(g.xsc2 + slot);
+  };
+  for (int i = threadIdx.x; i < hs; i += W * kSlice) {
+    const auto q = G(in.light + (size_t)G(g.sh_v)[hb + i] * L_N);
+    halo[3 * i + 0] = mk2(q[0], q[1]);
+    halo[3 * i + 1] = mk2(q[2], q[3]);
+    halo[3 * i + 2] = mk2(q[4], q[5]);
+  }
+  const Light<R> self = load_light(in.light, c);
+  R acc = R(0);
+  if (g.nbf > 0 && live && wv < 5 && has_boundary(g, P, c)) acc = G(w.bacc)[(size_t)wv * ncv + c];
+  // rows k .. k + W - 1 of component wv, in order, of the lanes with n rows. A
+  // group's box is written again two groups later, behind the next group's barrier.
+  auto add_rows = [&](const R(&b)[W][5][kSlice], int k, int n) {
+    lds_barrier();
+    if (W > 5 && wv >= 5) return;
+    R v[W];
+#pragma unroll
+    for (int r = 0; r < W; ++r) v[r] = b[r][wv][lane];
+#pragma unroll
+    for (int r = 0; r < W; ++r) {
+      const R sum = acc + pinned(v[r]);
+      acc = k + r < n ? sum : acc;
+    }
+  };
+  // compact pairs: their fluxes, signed for the cell
+  for (int k0 = 0; k0 < ncrow; k0 += kC * W) {
+    int code[kC];
+    R F[kC][5];
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+      const int k = k0 + j * W + wv;
+      code[j] = ldnt(g.cf_pair + cp0 + (k < ncrow ? k : ncrow - 1) * kSlice + (k < nc ? lane : 0));
+    }
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+      const int f = k0 + j * W + wv < nc ? code[j] & 0x7fffffff : 0;
+      const auto fl = G(w.cflux + (size_t)f * 6);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) F[j][q] = fl[q];
+    }
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+#pragma unroll
+      for (int q = 0; q < 5; ++q) box[j & 1][wv][q][lane] = flip(F[j][q], code[j] >= 0);
+      add_rows(box[j & 1], k0 + j * W, nc);
+    }
+  }
+  if (ncrow == 0) lds_barrier();  // the halo is staged
+  // extended rows, W at a time, the next W rows' loads in flight meanwhile
+  if (nrow > 0) {
+    auto group = [&](const Row& row, int ch, R(&b)[W][5][kSlice]) {
+      const int li = row.code & 0x7fff;
+      const T2 r0 = halo[3 * li + 0], r1 = halo[3 * li + 1], r2 = halo[3 * li + 2];
+      Light<R> other;
+      other.u[0] = r0.x; other.u[1] = r0.y; other.u[2] = r1.x; other.spv = r1.y; other.p = r2.x; other.h = r2.y;
+      other.rho = R(0); other.sos = R(0);
+      R F[5];
+      half_face_flux(F, row.n, row.cv, self, other, (row.code & 0x8000) != 0);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) b[wv][q][lane] = F[q];
+      add_rows(b, ch * W, deg);
+    };
+    Row ra, rb;
+    ld_row(ra, wv);
+    ld_row(rb, wv + W);
+    const int ngrp = (nrow + W - 1) / W;
+    for (int ch = 0; ch < ngrp; ch += 2) {
+      const int k = ch * W + wv;
+      group(ra, ch, box[0]);
+      ld_row(ra, k + 2 * W);
+      group(rb, ch + 1, box[1]);
+      ld_row(rb, k + 3 * W);
+    }
+  }
+  if (W == 5 || wv < 5) fin[wv][lane] = acc;
+  lds_barrier();
+  if (wv != 0 || !live) return;
+  R a5[5];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) a5[q] = fin[q][lane];
+  if (MODE == 0) {
+    write_rhs(rhs_out, ncv, c, a5, P);
+    return;
+  }
+  rk_update<STAGE>(g, in, out, w, P, c, self, a5);
 }
 
 // rk3Step of one stage from a stage RHS held in device memory, FP64 [5][ncv] in
@@ -2857,6 +3204,27 @@ inline int check() { return (int)hipGetLastError(); }
 
 namespace cgk {
 
+// Which flux pass a launch of nblk cell blocks takes (all give the same bits).
+// Row-split while every slice's workgroup is resident at once (3 per CU in FP64,
+// 6 in mixed precision: 192 and 384 blocks on 256 CUs); beyond that its halos and
+// barriers cost more than its parallelism gives. Ten wavefronts per slice while
+// there is at most one slice per CU. Measured us/step, thread per cell (pipelined)
+// against row-split, jittered boxes: FP64 24^3 (54 blocks) 272 / 162, 32^3 (128)
+// 276 / 230, 36^3 (183) 307 / 311, 40^3 (250) 341 / 418; mixed 32^3 198 / 154,
+// 40^3 240 / 223, 44^3 (333) 304 / 295, 56^3 (686) 488 / 500. Five against ten
+// wavefronts: FP64 16^3 158 / 143, 24^3 177 / 163, 28^3 (86) 212 / 217; mixed 24^3
+// 129 / 118, 32^3 154 / 153.
+template <class R>
+constexpr int kRowsBlocks = kMixed<R> ? 384 : 192;
+constexpr int kRows10Blocks = 64;
+// Thread per cell: pipelined loads up to 4 blocks per CU, where the wavefronts are
+// too few to hide a batch's round trip (flux pass, plain / pipelined: twelve solves
+// of 590 blocks 179 / 158 us FP64, 64^3 mixed 138 / 125 us). On larger launches
+// memory is busy anyway and the deeper queues only evict more of what the
+// wavefronts share in L2 (96^3, 3456 blocks: 740 / 758 us FP64, 400 / 424 mixed).
+constexpr int kPipeBlocks = 1024;
+static_assert(kRowsBlocks<float> <= kRowsMaxBlocks && kRowsBlocks<double> <= kRowsMaxBlocks, "slices' halos");
+
 template <class R>
 int launch_flux(int stage, int mode, const Launch<R>& L, int cur, double* rhs_out, void* stream) {
   if (launch_flux_compact(L, cur, stream)) return -1;
@@ -2901,6 +3269,32 @@ int launch_flux_ext(int stage, int mode, const Launch<R>& L, int cur, double* rh
   if (mode == 1 && L.zsum) {
     hipLaunchKernelGGL(k_zone_sums<R>, dim3(L.ninst), dim3(kBlock), 0, s, L.I, cur, stage);
     if (int rc = check()) return rc;
+  }
+  const bool rows = L.slds && L.nblk <= kRowsBlocks<R>, pipe = L.lds && L.nblk <= kPipeBlocks;
+  if (L.boundary && (rows || pipe)) {
+    hipLaunchKernelGGL(k_bflux<R>, grid, block, 0, s, L.I, L.bmap, cur, mode == 0 ? 1 : stage, mode);
+    if (int rc = check()) return rc;
+  }
+  if (rows) {
+    const dim3 sgrid(slice_grid(L.nblk));
+    auto go = [&](auto waves) {
+      constexpr int W = decltype(waves)::value;
+      const dim3 sblock(W * kSlice);
+      if (mode == 0) hipLaunchKernelGGL((k_flux_rows<R, 1, 0, W>), sgrid, sblock, L.slds, s, L.I, L.bmap, L.nblk, cur, rhs_out);
+      else if (stage == 1) hipLaunchKernelGGL((k_flux_rows<R, 1, 1, W>), sgrid, sblock, L.slds, s, L.I, L.bmap, L.nblk, cur, rhs_out);
+      else if (stage == 2) hipLaunchKernelGGL((k_flux_rows<R, 2, 1, W>), sgrid, sblock, L.slds, s, L.I, L.bmap, L.nblk, cur, rhs_out);
+      else hipLaunchKernelGGL((k_flux_rows<R, 3, 1, W>), sgrid, sblock, L.slds, s, L.I, L.bmap, L.nblk, cur, rhs_out);
+    };
+    if (L.nblk <= kRows10Blocks) go(std::integral_constant<int, 10>());
+    else go(std::integral_constant<int, 5>());
+    return check();
+  }
+  if (pipe) {
+    if (mode == 0) hipLaunchKernelGGL((k_flux_pipe<R, 1, 0>), grid, block, L.lds, s, L.I, L.bmap, cur, rhs_out);
+    else if (stage == 1) hipLaunchKernelGGL((k_flux_pipe<R, 1, 1>), grid, block, L.lds, s, L.I, L.bmap, cur, rhs_out);
+    else if (stage == 2) hipLaunchKernelGGL((k_flux_pipe<R, 2, 1>), grid, block, L.lds, s, L.I, L.bmap, cur, rhs_out);
+    else hipLaunchKernelGGL((k_flux_pipe<R, 3, 1>), grid, block, L.lds, s, L.I, L.bmap, cur, rhs_out);
+    return check();
   }
   if (L.lds) {
     auto go = [&](auto nb) {

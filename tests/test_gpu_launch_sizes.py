@@ -1,0 +1,52 @@
+"""The passes a step is made of are chosen by the launch's size (row-split,
+pipelined and plain kernels, with LDS halos); the batch option lds=0 keeps the
+plain global-gather kernels at every size. All add in the same order, so state
+and scalars must be the same bits on both sides of every size rule: one cell
+block, partly filled slices and blocks, and the blocks around each limit."""
+import numpy as np
+import pytest
+
+from nextgen_amd.batch import Batch, Instance, Layout
+from nextgen_amd.ic import tgv_params
+from nextgen_amd.ideal_gas import CG_PREC_FP64, CG_PREC_MIXED, Mesh, parse_params
+
+pytestmark = pytest.mark.gpu
+
+WALLS = ("y0 CBC_UPT 0.1 0.4 0 71.42857142857143 1.0\ny1 NSCBC_OUTLET_P 71.07 0.3 6.28\n")
+
+
+def states(mesh, prec, text, lds):
+    b = Batch(prec)
+    b.set_option("lds", lds)
+    b.set_option("graph", 0)
+    x = Instance(mesh, parse_params(text), *mesh.ic_tgv(0.1, 1.4), layout=Layout(mesh, prec))
+    i = b.attach(x)
+    b.step(3)
+    out = b.state(i), b.diag(i)
+    b.close()
+    return out
+
+
+# cells (blocks of 256): 343 (2), 4080 (16), 16250 (64), 16900 (67), 47952 (188),
+# 49284 (193), 97336 (381), 99452 (389), 262144 (1024), 266240 (1040)
+@pytest.mark.parametrize("prec", [CG_PREC_FP64, CG_PREC_MIXED])
+@pytest.mark.parametrize("kind,dims,sgs", [
+    ("jittered", (7, 7, 7), "VREMAN"), ("jittered", (17, 16, 15), "SIGMA"), ("jittered", (26, 25, 25), "VREMAN"),
+    ("jittered", (26, 26, 25), "NONE"), ("jittered", (37, 36, 36), "DSM_LOCAL"), ("jittered", (37, 37, 36), "VREMAN"),
+    ("jittered", (46, 46, 46), "VREMAN"), ("jittered", (47, 46, 46), "VREMAN"), ("lattice", (64, 64, 64), "NONE"),
+    ("lattice", (65, 64, 64), "NONE"), ("channel", (9, 11, 8), "VREMAN"), ("channel", (30, 28, 21), "VREMAN"),
+    ("channel", (40, 38, 35), "NONE")])
+def test_size_rules_bitwise(prec, kind, dims, sgs):
+    if kind == "lattice":
+        mesh = Mesh.lattice(dims)
+    elif kind == "channel":
+        mesh = Mesh.channel(dims, jitter=0.3, seed=5)
+    else:
+        mesh = Mesh.jittered(dims, 0.3, seed=5)
+    text = tgv_params(sgs=sgs) + f"PRECISION {'MIXED' if prec == CG_PREC_MIXED else 'FP64'}\n"
+    if kind == "channel":
+        text += WALLS
+    (a, da), (b, db) = states(mesh, prec, text, 1), states(mesh, prec, text, 0)
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(x, y)
+    assert da.cfl_max == db.cfl_max and da.dt == db.dt
