@@ -90,13 +90,19 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* G(T* p) {
   return (__attribute__((address_space(1))) T*)p;
 }
 
-// Running maximum of non-negative doubles by their bit patterns. The atomic
-// goes through a global-address-space pointer so that the compiler combines
-// the lanes of a wavefront into one atomic (a flat atomic would stay one per
-// lane, all on the same address).
+// Running maximum of non-negative doubles by their bit patterns. Atomics on one
+// address are taken one after the other (about 17 ns each over the chip), so the
+// value is read first and most callers, below the maximum so far, issue none.
 __device__ __forceinline__ void cfl_max(unsigned long long* p, unsigned long long v) {
-  __hip_atomic_fetch_max((__attribute__((address_space(1))) unsigned long long*)p, v, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+  const auto q = (__attribute__((address_space(1))) unsigned long long*)p;
+  if (v > __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    __hip_atomic_fetch_max(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the same of a wavefront's values, by one lane (all lanes active)
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+  for (int off = kSlice / 2; off > 0; off >>= 1) v = smax(v, __shfl_xor(v, off));
+  return v;
 }
 
 // Instance and instance-local block of this workgroup, or null for an empty
@@ -414,7 +420,10 @@ __device__ __forceinline__ void rk_update(const Geom& g, const State& in, const 
   const Light<double> L = eos(P, rho, u, rhoE, T);
   store_light(out.light, c, L);
   G(out.rhoE)[c] = rhoE;
-  if (STAGE == 3) G(w.logp)[c] = log(L.p * P.inv_pref);
+  if (STAGE == 3) {
+    G(w.thermo)[2 * (size_t)c] = log(L.p * P.inv_pref);
+    G(w.thermo)[2 * (size_t)c + 1] = 1.0 / (P.R_gas * T);
+  }
 }
 
 // Mixed precision: FP32 registers (energy row gauged), FP64 combination,
@@ -1999,7 +2008,8 @@ __global__ __launch_bounds__(kBlock) void k_eos(const Inst<R>* __restrict__ I, c
     const Light<double> in = load_light(st.light, c);
     const Light<double> L = eos(P, in.rho, in.u, G(st.rhoE)[c], T);
     store_light(st.light, c, L);
-    G(w.logp)[c] = log(L.p * P.inv_pref);
+    G(w.thermo)[2 * (size_t)c] = log(L.p * P.inv_pref);
+    G(w.thermo)[2 * (size_t)c + 1] = 1.0 / (P.R_gas * T);
   }
 }
 
@@ -2466,43 +2476,13 @@ __global__ __launch_bounds__(kBlock) void k_sensor_full(const Inst<R>* __restric
   G(w.vv2)[c] = double(vv2);
 }
 
-template <class R, int FIELDS, bool LDS>
-__global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
-                                                  int cur) {
-  int lblk;
-  const Inst<R>* Xp = inst_of(I, bmap, lblk);
-  if (!Xp) return;
-  const Inst<R>& X = *Xp;
-  const GeomT<R> g = X.g;
-  const StateT<R> st = X.st[cur];
-  const WorkT<R> w = X.w;
-  const Params& P = X.P;
+// The properties of one cell from its own state and velocity gradient: SGS
+// coefficients and material properties, written to its aux record (all but fgr).
+template <class R, int FIELDS>
+__device__ __forceinline__ void props_cell(const GeomT<R>& g, const WorkT<R>& w, const Params& P, int c,
+                                           const Light<R>& self) {
   const R Rg = R(P.R_gas);
   const R pg = kMixed<R> ? R(P.p_g) : R(0);
-  // per-cell terms of the Gibbs remainder, evaluated once per cell instead of
-  // once per half-face: 1/(R T) = 1/(R (p / (rho R))), and the last one
-  // ln p (FP64) or 1/p with p absolute (mixed precision)
-  auto irt_of = [&](R pp, R rr) { return mdiv(R(1), Rg * mdiv(kMixed<R> ? pp + pg : pp, rr * Rg)); };
-  extern __shared__ __align__(16) unsigned char smem[];
-  R* hrec = reinterpret_cast<R*>(smem);  // [hsize][4]: p, sp_vol, 1/(R T), ln p | 1/p
-  if constexpr (LDS) {
-    const int hb = G(g.halo_ptr)[lblk], hs = G(g.halo_ptr)[lblk + 1] - hb;
-    for (int i = threadIdx.x; i < hs; i += kBlock) {
-      const int gc = G(g.halo_v)[hb + i];
-      const auto q = G(st.light + (size_t)gc * L_N);
-      const R qp = q[L_P];
-      hrec[4 * i + 0] = qp;
-      hrec[4 * i + 1] = q[L_SPV];
-      hrec[4 * i + 2] = irt_of(qp, q[L_RHO]);
-      if constexpr (kMixed<R>) hrec[4 * i + 3] = mdiv(R(1), qp + pg);
-      else hrec[4 * i + 3] = G(w.logp)[gc];
-    }
-    __syncthreads();
-  }
-  const int pos = lblk * kBlock + threadIdx.x;
-  if (pos >= g.ncv) return;
-  const int c = cell_at(g.xperm, pos);
-  const Light<R> self = load_light(st.light, c);
   const R rho = self.rho, sos = self.sos;
   const R p = kMixed<R> ? self.p + pg : self.p;  // absolute pressure
   const R* u = self.u;
@@ -2573,104 +2553,9 @@ __global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I,
   const R symp = smax(R(P.coeff_p) * R(G(g.dcmag)[c]) * lambda / sos2 - R(G(g.dx23)[c]) * a_sgs, R(0));
   const R symh = R(P.coeff_h) * R(G(g.dcmag)[c]);
 
-  // ---- Gibbs-remainder sensor and convective CFL over the extended half-faces ----
-  const int lane = pos & (kSlice - 1);
-  const int cbase = G(g.cf_ptr)[pos >> 6] + lane;
-  const int xbase = G(g.xf_ptr)[pos >> 6] + lane;
-  const int nc = G(g.ef_nc)[pos];
-  const int nx = G(g.xf_deg)[pos];
-  // own ln p (FP64) or 1/p (mixed), as staged for the halo
-  const R l4_s = kMixed<R> ? mdiv(R(1), self.p + pg) : R(G(w.logp)[c]);
-  const R irt_s = irt_of(self.p, rho);  // 1 / (R T), as for the halo
-  R vv2 = R(0), cfl = boundary_cfl(g, c, self);
-  // Gibbs remainder of one pair from the neighbour's p, sp_vol, 1/(R T) and
-  // ln p (FP64: ln p1 - ln p0) or 1/p (mixed: log1p((p1 - p0) / p0))
-  auto gibbs = [&](R op, R ospv, R irt_o, R o4, bool self_hi) {
-    const R ap = self_hi ? op : self.p, bp = self_hi ? self.p : op;
-    const R aspv = self_hi ? ospv : self.spv, bspv = self_hi ? self.spv : ospv;
-    const R dp = bp - ap;
-    const R v_avg = R(0.5) * (aspv + bspv);
-    const R beta_avg = R(0.5) * ((self_hi ? irt_o : irt_s) + (self_hi ? irt_s : irt_o));
-    R gr;
-    if constexpr (kMixed<R>) gr = mlog1p(dp * (self_hi ? o4 : l4_s)) - v_avg * dp * beta_avg;
-    else gr = (self_hi ? l4_s : o4) - (self_hi ? o4 : l4_s) - v_avg * dp * beta_avg;
-    vv2 = smax(vv2, mabs(gr));
-  };
-  // compact pairs: sensor and CFL (the CFL sum in pair order). Slots are
-  // taken kQ at a time: their codes, then the neighbours' records and the face
-  // normals of all kQ, so the dependent gathers of different slots overlap.
-  constexpr int kQ = 2;
-  for (int k0 = 0; k0 < nc; k0 += kQ) {
-    int code[kQ];
-    R n[kQ][3];
-#pragma unroll
-    for (int j = 0; j < kQ; ++j)
-      if (k0 + j < nc) {
-        const int slot = cbase + (k0 + j) * kSlice;
-        code[j] = ldnt(g.cf_nbr + slot);
-        n[j][0] = ldnt(g.cfn0 + slot);
-        n[j][1] = ldnt(g.cfn1 + slot);
-        n[j][2] = ldnt(g.cfn2 + slot);
-      }
-    Light<R> o[kQ];
-    R l4[kQ];
-#pragma unroll
-    for (int j = 0; j < kQ; ++j)
-      if (k0 + j < nc) {
-        const int nb = code[j] & 0x7fffffff;
-        o[j] = load_light(st.light, nb);
-        if constexpr (!kMixed<R>) l4[j] = G(w.logp)[nb];
-      }
-#pragma unroll
-    for (int j = 0; j < kQ; ++j) {
-      if (k0 + j >= nc) break;
-      const bool self_hi = code[j] < 0;
-      const Light<R>& oj = o[j];
-      if (!P.full_gr) gibbs(oj.p, oj.spv, irt_of(oj.p, oj.rho), kMixed<R> ? mdiv(R(1), oj.p + pg) : l4[j], self_hi);
-      const Light<R>& a = self_hi ? oj : self;
-      const Light<R>& b = self_hi ? self : oj;
-      const R* nj = n[j];
-      const R area = msqrt(nj[0] * nj[0] + nj[1] * nj[1] + nj[2] * nj[2]);
-      const R undA = R(0.5) * ((a.u[0] * nj[0] + a.u[1] * nj[1] + a.u[2] * nj[2]) +
-                               (b.u[0] * nj[0] + b.u[1] * nj[1] + b.u[2] * nj[2]));
-      const R sos_avg = R(0.5) * (a.sos + b.sos);
-      cfl += mabs(undA) + area * sos_avg;
-    }
-  }
-  // purely extended pairs: sensor only (a maximum: order-independent); their
-  // codes are fetched kP at a time so the loads overlap
-  constexpr int kP = 8;
-  // (with USE_FULL_GR the sensor maximum comes from k_sensor_full instead)
-  if (P.full_gr) vv2 = R(G(w.vv2)[c]);
-  for (int k0 = 0; k0 < (P.full_gr ? 0 : nx); k0 += kP) {
-    int code[kP];
-#pragma unroll
-    for (int j = 0; j < kP; ++j)
-      if (k0 + j < nx) code[j] = LDS ? int(ldnt(g.xf_loc + xbase + (k0 + j) * kSlice)) : ldnt(g.xf_nbr + xbase + (k0 + j) * kSlice);
-#pragma unroll
-    for (int j = 0; j < kP; ++j) {
-      if (k0 + j >= nx) break;
-      if constexpr (LDS) {
-        const R* h = hrec + 4 * (code[j] & 0x7fff);
-        gibbs(h[0], h[1], h[2], h[3], (code[j] & 0x8000) != 0);
-      } else {
-        const int nb = code[j] & 0x7fffffff;
-        const auto q = G(st.light + (size_t)nb * L_N);
-        const R qp = q[L_P];
-        gibbs(qp, q[L_SPV], irt_of(qp, q[L_RHO]), kMixed<R> ? mdiv(R(1), qp + pg) : R(G(w.logp)[nb]), code[j] < 0);
-      }
-    }
-  }
-  R fgr;
-  if (P.diss_mode == 1 && !P.full_gr) fgr = R(0);  // setFgrCvsFull has no NO_DISS / ALL_DISS
-  else if (P.diss_mode == 2 && !P.full_gr) fgr = R(0.5);
-  else fgr = R(0.5) / (R(1) + mexp(R(-2) * (vv2 - R(P.gr_nrm)) / R(5.0e-03)));
-  cfl *= R(0.5) * R(1) * R(G(g.inv_vol)[c]);
-
   auxc[A_MU] = mu_lam + mu_sgs;
   auxc[A_LOC] = loc_lam + loc_sgs;
   auxc[A_ASGS] = a_sgs;
-  auxc[A_FGR] = fgr;
   auxc[A_SYMH] = symh;
   auxc[A_SYMP] = symp;
   if (FIELDS) {
@@ -2680,10 +2565,324 @@ __global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I,
     G(w.loc_lam)[c] = loc_lam;
     G(w.loc_sgs)[c] = loc_sgs;
     G(w.a_sgs)[c] = a_sgs;
-    G(w.vv2)[c] = vv2;
   }
-  if (cfl == cfl) cfl_max(&w.info->cfl_bits, (unsigned long long)__double_as_longlong(double(cfl)));
   if (rho != rho || p != p || T != T) G(w.info)->nan = 1;
+}
+
+// What a cell's sensor and CFL sums give: fgr from the Gibbs remainder's maximum,
+// and the convective CFL at dt = 1
+template <class R, int FIELDS>
+__device__ __forceinline__ void props_sensor(const GeomT<R>& g, const WorkT<R>& w, const Params& P, int c, R vv2) {
+  R fgr;
+  if (P.diss_mode == 1 && !P.full_gr) fgr = R(0);  // setFgrCvsFull has no NO_DISS / ALL_DISS
+  else if (P.diss_mode == 2 && !P.full_gr) fgr = R(0.5);
+  else fgr = R(0.5) / (R(1) + mexp(R(-2) * (vv2 - R(P.gr_nrm)) / R(5.0e-03)));
+  G(w.aux + (size_t)c * A_N)[A_FGR] = fgr;
+  if (FIELDS) G(w.vv2)[c] = vv2;
+}
+// (a NaN does not count)
+template <class R>
+__device__ __forceinline__ double props_cfl(const GeomT<R>& g, int c, R cfl) {
+  cfl *= R(0.5) * R(1) * R(G(g.inv_vol)[c]);
+  return cfl == cfl ? double(cfl) : 0.0;
+}
+
+// Per-cell terms of the Gibbs remainder: p, sp_vol, 1/(R T) = 1/(R (p / (rho R)))
+// and ln p (FP64) or 1/p with p absolute (mixed precision). In FP64 the last two
+// are kept per cell (w.thermo, with the state), in mixed precision formed here.
+template <class R>
+struct Gibbs {
+  R p, spv, irt, l4;
+};
+template <class R>
+__device__ __forceinline__ Gibbs<R> gibbs_of(const WorkT<R>& w, R Rg, R pg, R p, R spv, R rho, int c) {
+  if constexpr (kMixed<R>) return {p, spv, mdiv(R(1), Rg * mdiv(p + pg, rho * Rg)), mdiv(R(1), p + pg)};
+  else return {p, spv, G(w.thermo)[2 * (size_t)c + 1], G(w.thermo)[2 * (size_t)c]};
+}
+// |Gibbs remainder| of one pair: with dp = p1 - p0 along the pair,
+//   FP64  ln p1 - ln p0 - v_avg dp beta_avg: every term changes sign exactly with
+//         the orientation, so the magnitude needs none;
+//   mixed log1p((p1 - p0) / p0) - v_avg dp beta_avg.
+template <class R>
+__device__ __forceinline__ R gibbs_abs(const Gibbs<R>& s, const Gibbs<R>& o, bool self_hi) {
+  R dp = o.p - s.p;
+  const R v_avg = R(0.5) * (s.spv + o.spv);
+  const R beta_avg = R(0.5) * (s.irt + o.irt);
+  R gr;
+  if constexpr (kMixed<R>) {
+    dp = flip(dp, self_hi);
+    gr = mlog1p(dp * (self_hi ? o.l4 : s.l4)) - v_avg * dp * beta_avg;
+  } else {
+    gr = o.l4 - s.l4 - v_avg * dp * beta_avg;
+  }
+  return mabs(gr);
+}
+// One compact face's term of the convective CFL sum
+template <class R>
+__device__ __forceinline__ R cfl_term(const R n[3], const Light<R>& self, const Light<R>& o, bool self_hi) {
+  const R area = msqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+  const R us = self.u[0] * n[0] + self.u[1] * n[1] + self.u[2] * n[2];
+  const R uo = o.u[0] * n[0] + o.u[1] * n[1] + o.u[2] * n[2];
+  const R undA = R(0.5) * (us + uo);
+  const R sos_avg = R(0.5) * (self.sos + o.sos);
+  return mabs(undA) + area * sos_avg;
+}
+
+// Properties pass, thread per cell. In mixed precision it was bound by one CFL
+// atomic per wavefront on one address; with one per block that raises the maximum
+// 96^3 cells take 166 us (233), 64^3 62 us (97). FP64 (289 us, 285) is bound by
+// its gathers: 2.2 GB per 2.1M cells at 3.5 TB/s.
+template <class R, int FIELDS, bool LDS>
+__global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
+                                                  int cur) {
+  int lblk;
+  const Inst<R>* Xp = inst_of(I, bmap, lblk);
+  if (!Xp) return;
+  const Inst<R>& X = *Xp;
+  const GeomT<R> g = X.g;
+  const StateT<R> st = X.st[cur];
+  const WorkT<R> w = X.w;
+  const Params& P = X.P;
+  const R Rg = R(P.R_gas);
+  const R pg = kMixed<R> ? R(P.p_g) : R(0);
+  extern __shared__ __align__(16) unsigned char smem[];
+  Gibbs<R>* hrec = reinterpret_cast<Gibbs<R>*>(smem);  // [hsize]
+  if constexpr (LDS) {
+    const int hb = G(g.halo_ptr)[lblk], hs = G(g.halo_ptr)[lblk + 1] - hb;
+    for (int i = threadIdx.x; i < hs; i += kBlock) {
+      const int gc = G(g.halo_v)[hb + i];
+      const auto q = G(st.light + (size_t)gc * L_N);
+      hrec[i] = gibbs_of(w, Rg, pg, q[L_P], q[L_SPV], q[L_RHO], gc);
+    }
+    __syncthreads();
+  }
+  const int pos = lblk * kBlock + threadIdx.x;
+  double cfl_cell = 0.0;
+  if (pos < g.ncv) {
+    const int c = cell_at(g.xperm, pos);
+    const Light<R> self = load_light(st.light, c);
+    props_cell<R, FIELDS>(g, w, P, c, self);
+
+    // ---- Gibbs-remainder sensor and convective CFL over the extended half-faces ----
+    const int lane = pos & (kSlice - 1), sl = pos >> 6;
+    const int cp0 = G(g.cf_ptr)[sl], ncrow = (G(g.cf_ptr)[sl + 1] - cp0) / kSlice;
+    const int xp0 = G(g.xf_ptr)[sl], nrow = (G(g.xf_ptr)[sl + 1] - xp0) / kSlice;
+    const int nc = G(g.ef_nc)[pos];
+    const int nx = G(g.xf_deg)[pos];
+    const Gibbs<R> gs = gibbs_of(w, Rg, pg, self.p, self.spv, self.rho, c);
+    R vv2 = R(0), cfl = boundary_cfl(g, c, self);
+    // No load below is under a branch, so that a wait for one batch leaves the next
+    // in flight: a lane past its last row reads its slice's first slot of the row,
+    // a line that is fetched anyway, and its terms are not used.
+    // Compact pairs: sensor and CFL (the CFL sum in pair order), kQ rows at a time:
+    // their codes and face normals, then the neighbours' records.
+    constexpr int kQ = 2;
+    if (ncrow > 0) {
+      int code[kQ];
+      R n[kQ][3];
+      auto ld = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          const int k = k0 + j;
+          const int slot = cp0 + (k < ncrow ? k : ncrow - 1) * kSlice + (k < nc ? lane : 0);
+          code[j] = ldnt(g.cf_nbr + slot);
+          n[j][0] = ldnt(g.cfn0 + slot);
+          n[j][1] = ldnt(g.cfn1 + slot);
+          n[j][2] = ldnt(g.cfn2 + slot);
+        }
+      };
+      ld(0);
+      for (int k0 = 0; k0 < ncrow; k0 += kQ) {
+        Light<R> o[kQ];
+        Gibbs<R> go[kQ];
+        R nn[kQ][3];
+        bool hi[kQ];
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          hi[j] = code[j] < 0;
+          const int nb = code[j] & 0x7fffffff;
+          o[j] = load_light(st.light, nb);
+          go[j] = gibbs_of(w, Rg, pg, o[j].p, o[j].spv, o[j].rho, nb);
+          nn[j][0] = n[j][0]; nn[j][1] = n[j][1]; nn[j][2] = n[j][2];
+        }
+        ld(k0 + kQ);
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          const bool on = k0 + j < nc;
+          const R v = smax(vv2, gibbs_abs(gs, go[j], hi[j]));
+          vv2 = on ? v : vv2;
+          const R sum = cfl + cfl_term(nn[j], self, o[j], hi[j]);
+          cfl = on ? sum : cfl;
+        }
+      }
+    }
+    // Purely extended pairs: sensor only (a maximum: order-independent); kP codes at
+    // a time, the next ones while these are used. With USE_FULL_GR the sensor
+    // maximum comes from k_sensor_full instead.
+    constexpr int kP = 8;
+    if (P.full_gr) {
+      vv2 = R(G(w.vv2)[c]);
+    } else if (nrow > 0) {
+      int code[kP];
+      auto ld = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+          const int k = k0 + j;
+          const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < nx ? lane : 0);
+          code[j] = LDS ? int(ldnt(g.xf_loc + slot)) : ldnt(g.xf_nbr + slot);
+        }
+      };
+      ld(0);
+      for (int k0 = 0; k0 < nrow; k0 += kP) {
+        int cc[kP];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) cc[j] = code[j];
+        ld(k0 + kP);
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+          Gibbs<R> o;
+          bool hi;
+          if constexpr (LDS) {
+            o = hrec[cc[j] & 0x7fff];
+            hi = (cc[j] & 0x8000) != 0;
+          } else {
+            const int nb = cc[j] & 0x7fffffff;
+            const auto q = G(st.light + (size_t)nb * L_N);
+            o = gibbs_of(w, Rg, pg, q[L_P], q[L_SPV], q[L_RHO], nb);
+            hi = cc[j] < 0;
+          }
+          const R v = smax(vv2, gibbs_abs(gs, o, hi));
+          vv2 = k0 + j < nx ? v : vv2;
+        }
+      }
+    }
+    props_sensor<R, FIELDS>(g, w, P, c, vv2);
+    cfl_cell = props_cfl(g, c, cfl);
+  }
+  // the block's CFL maximum, one atomic
+  __shared__ double wmax[kBlock / kSlice];
+  const double m = wave_max(cfl_cell);
+  if ((threadIdx.x & (kSlice - 1)) == 0) wmax[threadIdx.x / kSlice] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double bm = wmax[0];
+#pragma unroll
+    for (int i = 1; i < kBlock / kSlice; ++i) bm = smax(bm, wmax[i]);
+    cfl_max(&w.info->cfl_bits, (unsigned long long)__double_as_longlong(bm));
+  }
+}
+
+// The properties pass split by rows, for the launches of the row-split flux pass
+// (see k_flux_rows; 16^3 mixed 32 -> 12 us, 32^3 FP64 43 -> 24 us): one workgroup of 5 wavefronts per slice. Wavefronts 0-3 share
+// the rows; the last computes the cells' own part meanwhile.
+template <class R, int FIELDS>
+__global__ __launch_bounds__(5 * kSlice) void k_props_rows(const Inst<R>* __restrict__ I,
+                                                           const int* __restrict__ bmap, int nblk, int cur) {
+  constexpr int W = 4, kC = 4;
+  extern __shared__ __align__(16) unsigned char smem[];
+  Gibbs<R>* hrec = reinterpret_cast<Gibbs<R>*>(smem);  // [hsize]
+  __shared__ R box[kC][W][kSlice], mx[W][kSlice];
+  int pos0 = 0;
+  const Inst<R>* Xp = slice_of(I, bmap, nblk, pos0);
+  if (!Xp) return;
+  const Inst<R>& X = *Xp;
+  const GeomT<R> g = X.g;
+  const StateT<R> st = X.st[cur];
+  const WorkT<R> w = X.w;
+  const Params& P = X.P;
+  const R Rg = R(P.R_gas);
+  const R pg = kMixed<R> ? R(P.p_g) : R(0);
+  const int lane = threadIdx.x & (kSlice - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice);
+  const int pos = pos0 + lane;
+  const bool live = pos < g.ncv;
+  const int c = live ? cell_at(g.xperm, pos) : pos0;
+  const int sl = pos0 / kSlice;
+  const int cp0 = G(g.cf_ptr)[sl], ncrow = (G(g.cf_ptr)[sl + 1] - cp0) / kSlice;
+  const int xp0 = G(g.xf_ptr)[sl], nrow = (G(g.xf_ptr)[sl + 1] - xp0) / kSlice;
+  const int nc = live ? G(g.ef_nc)[pos] : 0, nx = live ? G(g.xf_deg)[pos] : 0;
+  const int hb = G(g.sh_ptr)[sl], hs = G(g.sh_ptr)[sl + 1] - hb;
+  for (int i = threadIdx.x; i < hs; i += (W + 1) * kSlice) {
+    const int gc = G(g.sh_v)[hb + i];
+    const auto q = G(st.light + (size_t)gc * L_N);
+    hrec[i] = gibbs_of(w, Rg, pg, q[L_P], q[L_SPV], q[L_RHO], gc);
+  }
+  const Light<R> self = load_light(st.light, c);
+  const Gibbs<R> gs = gibbs_of(w, Rg, pg, self.p, self.spv, self.rho, c);
+  R vv2 = R(0), cfl = R(0);
+  if (wv == W - 1 && live) cfl = boundary_cfl(g, c, self);
+  // compact rows: their CFL terms through LDS, added in pair order by wavefront W - 1
+  for (int k0 = 0; k0 < ncrow; k0 += kC * W) {
+    if (wv < W) {
+      int code[kC];
+      R n[kC][3];
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        const int k = k0 + j * W + wv;
+        const int slot = cp0 + (k < ncrow ? k : ncrow - 1) * kSlice + (k < nc ? lane : 0);
+        code[j] = ldnt(g.cf_nbr + slot);
+        n[j][0] = ldnt(g.cfn0 + slot);
+        n[j][1] = ldnt(g.cfn1 + slot);
+        n[j][2] = ldnt(g.cfn2 + slot);
+      }
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        const int nb = code[j] & 0x7fffffff;
+        const Light<R> o = load_light(st.light, nb);
+        const R v = smax(vv2, gibbs_abs(gs, gibbs_of(w, Rg, pg, o.p, o.spv, o.rho, nb), code[j] < 0));
+        vv2 = k0 + j * W + wv < nc ? v : vv2;
+        box[j][wv][lane] = cfl_term(n[j], self, o, code[j] < 0);
+      }
+    }
+    lds_barrier();
+    if (wv == W - 1) {
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        R v[W];
+#pragma unroll
+        for (int r = 0; r < W; ++r) v[r] = box[j][r][lane];
+#pragma unroll
+        for (int r = 0; r < W; ++r) {
+          const R sum = cfl + pinned(v[r]);
+          cfl = k0 + j * W + r < nc ? sum : cfl;
+        }
+      }
+    }
+    lds_barrier();
+  }
+  if (ncrow == 0) lds_barrier();  // the halo is staged
+  if (wv == W) {
+    if (live) props_cell<R, FIELDS>(g, w, P, c, self);
+  } else {
+    if (wv == W - 1) {
+      const double m = wave_max(live ? props_cfl(g, c, cfl) : 0.0);
+      if (lane == 0) cfl_max(&w.info->cfl_bits, (unsigned long long)__double_as_longlong(m));
+    }
+    if (P.full_gr) {
+      vv2 = R(G(w.vv2)[c]);
+    } else if (nrow > 0) {
+      constexpr int kP = 4;
+      for (int k0 = wv; k0 < nrow; k0 += kP * W) {
+        int code[kP];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+          const int k = k0 + j * W;
+          code[j] = ldnt(g.sh_loc + xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < nx ? lane : 0));
+        }
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+          const R v = smax(vv2, gibbs_abs(gs, hrec[code[j] & 0x7fff], (code[j] & 0x8000) != 0));
+          vv2 = k0 + j * W < nx ? v : vv2;
+        }
+      }
+    }
+    mx[wv][lane] = vv2;
+  }
+  lds_barrier();
+  if (wv != 0 || !live) return;
+#pragma unroll
+  for (int r = 1; r < W; ++r) vv2 = smax(vv2, mx[r][lane]);
+  props_sensor<R, FIELDS>(g, w, P, c, vv2);
 }
 
 // setDt (FlowSolver.hpp:2274-2328) and the step/time bookkeeping of
@@ -3352,6 +3551,12 @@ int launch_props(const Launch<R>& L, int cur, int fields, void* stream) {
   // mu_lam) every step
   const size_t lds = L.lds / 6 * 4;
   fields = (fields || L.scalars || L.boundary) ? 1 : 0;
+  if (L.slds && L.nblk <= kRowsBlocks<R>) {
+    const dim3 grid(slice_grid(L.nblk)), block(5 * kSlice);
+    if (fields) hipLaunchKernelGGL((k_props_rows<R, 1>), grid, block, L.slds / 6 * 4, s, L.I, L.bmap, L.nblk, cur);
+    else hipLaunchKernelGGL((k_props_rows<R, 0>), grid, block, L.slds / 6 * 4, s, L.I, L.bmap, L.nblk, cur);
+    return check();
+  }
   if (lds) {
     if (fields) hipLaunchKernelGGL((k_props<R, 1, true>), dim3(L.nblk), dim3(kBlock), lds, s, L.I, L.bmap, cur);
     else hipLaunchKernelGGL((k_props<R, 0, true>), dim3(L.nblk), dim3(kBlock), lds, s, L.I, L.bmap, cur);

@@ -27,11 +27,11 @@ def states(mesh, prec, text, lds):
     return out
 
 
-# cells (blocks of 256): 343 (2), 4080 (16), 16250 (64), 16900 (67), 47952 (188),
+# cells (blocks of 256): 576 (3), 4080 (16), 16250 (64), 16900 (67), 47952 (188),
 # 49284 (193), 97336 (381), 99452 (389), 262144 (1024), 266240 (1040)
 @pytest.mark.parametrize("prec", [CG_PREC_FP64, CG_PREC_MIXED])
 @pytest.mark.parametrize("kind,dims,sgs", [
-    ("jittered", (7, 7, 7), "VREMAN"), ("jittered", (17, 16, 15), "SIGMA"), ("jittered", (26, 25, 25), "VREMAN"),
+    ("jittered", (9, 8, 8), "VREMAN"), ("jittered", (17, 16, 15), "SIGMA"), ("jittered", (26, 25, 25), "VREMAN"),
     ("jittered", (26, 26, 25), "NONE"), ("jittered", (37, 36, 36), "DSM_LOCAL"), ("jittered", (37, 37, 36), "VREMAN"),
     ("jittered", (46, 46, 46), "VREMAN"), ("jittered", (47, 46, 46), "VREMAN"), ("lattice", (64, 64, 64), "NONE"),
     ("lattice", (65, 64, 64), "NONE"), ("channel", (9, 11, 8), "VREMAN"), ("channel", (30, 28, 21), "VREMAN"),
