@@ -198,6 +198,14 @@ struct Instance : HostInst {
   }
 };
 
+// A solver's or batch's pinned memory: its StepInfo mirror, then the landing place
+// of small device reads (a pageable destination costs the runtime a staging copy
+// and a wait per read)
+constexpr size_t kLanding = size_t(1) << 20;
+constexpr size_t kPinned = 256 + kLanding;
+static_assert(sizeof(cgdev::StepInfo) <= 256, "the mirror's place");
+inline double* landing(cgdev::StepInfo* info) { return reinterpret_cast<double*>(reinterpret_cast<char*>(info) + 256); }
+
 // instances of one precision advanced together
 template <class R>
 struct Engine {
@@ -226,7 +234,7 @@ struct Engine {
 struct cg_solver : Err {
   bool mixed = false;
   hipStream_t stream = nullptr;
-  cgdev::StepInfo* info_host = nullptr;  // pinned mirror
+  cgdev::StepInfo* info_host = nullptr;  // pinned mirror, first of kPinned bytes
   Engine<double> ed;
   Engine<float> ef;
   Instance<double>* id = nullptr;
@@ -556,6 +564,8 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
       std::stable_sort(ext_of.begin() + b0, ext_of.begin() + std::min(ncv, b0 + sort_group), [&](int a, int b) {
         return xcnt_m[a] != xcnt_m[b] ? xcnt_m[a] > xcnt_m[b] : ccnt_m[a] > ccnt_m[b];
       });
+  if (sort_group > 0)
+    if (int urc = upload(s, h, &g.ext, ext_of)) return urc;
   std::vector<int> int_of(ncv);
   for (int c = 0; c < ncv; ++c) int_of[ext_of[c]] = c;
   std::vector<double> inv_vol(ncv), vol(ncv), sa_to_vol(ncv), dcmag(ncv), dx13(ncv), dx23(ncv);
@@ -1040,7 +1050,7 @@ int build_instance(Err* s, Instance<R>* I, std::shared_ptr<Layout<R>> lay, const
   rc |= dev_alloc(s, h, &hi->info, 1);
   w.info = hi->info;
   rc |= dev_alloc(s, h, &w.partial, 8 * (size_t)hi->nblocks);
-  rc |= dev_alloc(s, h, &w.diag, 8);
+  rc |= dev_alloc(s, h, &w.diag, 9);
   hi->snap_n = mixed ? (size_t)ncv * 5 : (size_t)ncv * (cgdev::L_N + 1);
   if (hi->nscbc) {
     // NSCBC outlet faces: their states (in the snapshots too) and stage rates
@@ -1506,36 +1516,35 @@ int get_rec(Err* s, int ncv, const int* ext, const T* rec, int stride, int f0, i
   return 0;
 }
 
-template <class R>
-int get_state(Err* s, Instance<R>* I, int cur, double* rho, double* u, double* rhoE, hipStream_t stream) {
-  const cgdev::StateT<R>& st = I->b.st[cur];
-  const int ncv = I->ncv;
-  if constexpr (std::is_same<R, float>::value) {
-    const size_t n = (size_t)ncv;
-    double* cons = st.cons;
-    if (rho) {
-      double* f[1] = {cons};
-      if (int rc = get_soa(s, ncv, I->ext_of, f, 1, rho, stream)) return rc;
-    }
-    if (u) {
-      double* f[3] = {cons + n, cons + 2 * n, cons + 3 * n};
-      if (int rc = get_soa(s, ncv, I->ext_of, f, 3, u, stream)) return rc;
-    }
-    if (rhoE) {
-      double* f[1] = {cons + 4 * n};
-      if (int rc = get_soa(s, ncv, I->ext_of, f, 1, rhoE, stream)) return rc;
-    }
-  } else {
-    if (rho)
-      if (int rc = get_rec(s, ncv, I->ext_of, st.light, cgdev::L_N, cgdev::L_RHO, 1, rho, stream)) return rc;
-    if (u)
-      if (int rc = get_rec(s, ncv, I->ext_of, st.light, cgdev::L_N, cgdev::L_U0, 3, u, stream)) return rc;
-    if (rhoE) {
-      double* f[1] = {st.rhoE};
-      if (int rc = get_soa(s, ncv, I->ext_of, f, 1, rhoE, stream)) return rc;
-    }
+// n doubles from the device to out[i], len[i] each, one after the other (out[i]
+// null: not wanted), through the landing place where they fit
+int read_parts(Err* s, cgdev::StepInfo* info, const double* dev, int parts, double* const out[], const size_t len[],
+               hipStream_t stream) {
+  size_t n = 0;
+  for (int i = 0; i < parts; ++i) n += len[i];
+  if (n * sizeof(double) <= kLanding) {
+    double* land = landing(info);
+    HIPCHK(s, hipMemcpyAsync(land, dev, n * sizeof(double), hipMemcpyDeviceToHost, stream));
+    HIPCHK(s, hipStreamSynchronize(stream));
+    for (int i = 0; i < parts; land += len[i++])
+      if (out[i]) std::memcpy(out[i], land, len[i] * sizeof(double));
+    return 0;
   }
+  for (int i = 0; i < parts; dev += len[i++])
+    if (out[i]) HIPCHK(s, hipMemcpyAsync(out[i], dev, len[i] * sizeof(double), hipMemcpyDeviceToHost, stream));
+  HIPCHK(s, hipStreamSynchronize(stream));
   return 0;
+}
+
+template <class R>
+int get_state(Err* s, Instance<R>* I, int cur, cgdev::StepInfo* host, double* rho, double* u, double* rhoE,
+              hipStream_t stream) {
+  const size_t n = (size_t)I->ncv;
+  if (const int le = cgk::launch_pack_state(I->solo_launch(), I->ncv, cur, I->rhs_tmp, stream))
+    return launch_fail(s, "pack", le);
+  double* const out[3] = {rho, u, rhoE};
+  const size_t len[3] = {n, 3 * n, n};
+  return read_parts(s, host, I->rhs_tmp, 3, out, len, stream);
 }
 
 template <class R>
@@ -1552,9 +1561,13 @@ int calc_cfl(Err* s, Instance<R>* I, int cur, double dt, double* cfl_max, hipStr
 
 template <class R>
 int get_diag(Err* s, Instance<R>* I, int cur, cgdev::StepInfo* host, cg_diag* d, hipStream_t stream) {
-  if (const int le = cgk::launch_diag(I->solo_launch(), cur, stream)) return launch_fail(s, "diag", le);
-  double v[8];
-  HIPCHK(s, hipMemcpyAsync(v, I->b.w.diag, sizeof(v), hipMemcpyDeviceToHost, stream));
+  // the sums, the CFL maximum at the solve's dt and its StepInfo, in one wait
+  const cgk::Launch<R> L = I->solo_launch();
+  if (const int le = cgk::launch_diag(L, cur, stream)) return launch_fail(s, "diag", le);
+  if (const int le = cgk::launch_cfl(L, cur, 0.0, stream, reinterpret_cast<unsigned long long*>(I->b.w.diag + 8), true))
+    return launch_fail(s, "cfl", le);
+  double* v = landing(host);
+  HIPCHK(s, hipMemcpyAsync(v, I->b.w.diag, 9 * sizeof(double), hipMemcpyDeviceToHost, stream));
   if (int rc = read_info(s, I, host, stream)) return rc;
   d->step = host->step;
   d->time = host->time;
@@ -1563,9 +1576,7 @@ int get_diag(Err* s, Instance<R>* I, int cur, cgdev::StepInfo* host, cg_diag* d,
   d->enstrophy = v[6] / v[7];
   for (int q = 0; q < 5; ++q) d->sums[q] = v[q];
   d->nan_flag = host->nan;
-  double cm = 0.0;
-  if (int rc = calc_cfl(s, I, cur, d->dt, &cm, stream)) return rc;
-  d->cfl_max = cm;
+  d->cfl_max = v[8];
   return 0;
 }
 
@@ -2407,7 +2418,7 @@ int cg_create(const cg_mesh* m, const cg_params* p, cg_solver** out) {
   int count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count < 1) return bail(s->set(CG_EHIP, "no HIP device available"));
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess) return bail(s->set(CG_EHIP, "stream creation failed"));
-  if (hipHostMalloc((void**)&s->info_host, sizeof(cgdev::StepInfo)) != hipSuccess) return bail(s->set(CG_EHIP, "pinned alloc failed"));
+  if (hipHostMalloc((void**)&s->info_host, kPinned) != hipSuccess) return bail(s->set(CG_EHIP, "pinned alloc failed"));
   std::memset(s->info_host, 0, sizeof(cgdev::StepInfo));
   const bool lds = !std::getenv("CG_NO_LDS");
   int rc = 0;
@@ -2442,7 +2453,7 @@ int cg_set_state(cg_solver* s, const double* rho, const double* u, const double*
 
 int cg_get_state(cg_solver* s, double* rho, double* u, double* rhoE) {
   if (!s) return fail(CG_EINVAL, "null solver");
-  const int rc = with_inst(s, [&](auto& E, auto* I) { return get_state(s, I, E.cur, rho, u, rhoE, s->stream); });
+  const int rc = with_inst(s, [&](auto& E, auto* I) { return get_state(s, I, E.cur, s->info_host, rho, u, rhoE, s->stream); });
   return rc ? rc : CG_OK;
 }
 
@@ -2554,9 +2565,15 @@ int cg_calc_rhs(cg_solver* s, int stage, double* rhs) {
     if (!I->ready) return s->set(CG_ESTATE, "call cg_init_complete first");
     if (const int le = cgk::launch_flux(stage, 0, I->solo_launch(), E.cur, I->rhs_tmp, s->stream))
       return launch_fail(s, "flux", le);
-    double* f[5];
-    for (int q = 0; q < 5; ++q) f[q] = I->rhs_tmp + (size_t)q * I->ncv;
-    return get_soa(s, I->ncv, I->ext_of, f, 5, rhs, s->stream);
+    // to mesh order in the state buffer that no stage has written yet
+    const auto& spare = I->b.st[E.cur ^ 1];
+    double* packed = spare.cons;
+    if constexpr (!std::is_same<std::decay_t<decltype(*spare.light)>, float>::value) packed = spare.light;
+    if (const int le = cgk::launch_pack_rhs(I->solo_launch(), I->ncv, I->rhs_tmp, packed, s->stream))
+      return launch_fail(s, "pack", le);
+    double* const out[1] = {rhs};
+    const size_t len[1] = {5 * (size_t)I->ncv};
+    return read_parts(s, s->info_host, packed, 1, out, len, s->stream);
   });
 }
 
@@ -2686,7 +2703,7 @@ int cg_write_sles(cg_solver* s, const char* path) {
     if (!I->ready) return s->set(CG_ESTATE, "call cg_init_complete first");
     const size_t n = (size_t)I->ncv;
     std::vector<double> rho(n), u(3 * n), rhoE(n), p(n), T(n);
-    if (int rc = get_state(s, I, E.cur, rho.data(), u.data(), rhoE.data(), s->stream)) return rc;
+    if (int rc = get_state(s, I, E.cur, s->info_host, rho.data(), u.data(), rhoE.data(), s->stream)) return rc;
     if (int rc = cg_get_field(s, "p", p.data(), (int64_t)n)) return rc;
     if (int rc = cg_get_field(s, "T", T.data(), (int64_t)n)) return rc;
     if (int rc = read_info(s, I, s->info_host, s->stream)) return rc;
@@ -2922,7 +2939,7 @@ int cg_batch_create(int precision, cg_batch** out) {
   int count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count < 1 ||
       hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipHostMalloc((void**)&b->info_host, sizeof(cgdev::StepInfo)) != hipSuccess) {
+      hipHostMalloc((void**)&b->info_host, kPinned) != hipSuccess) {
     cg_batch_destroy(b);
     return fail(CG_EHIP, "no HIP device, stream or pinned memory");
   }
@@ -3139,13 +3156,30 @@ int cg_batch_step(cg_batch* b, int nsteps) {
       if (int rc = engine_steps(b, E, b->stream, chunk, b->use_graph)) return rc;
       it += chunk;
       for (auto* I : E.inst) I->host_step += chunk;
-      for (auto* I : E.inst) {
-        const int ci = std::max(1, I->prm.check_interval);
-        if (I->host_step % ci != 0 && it != nsteps) continue;
-        bool rolled = false;
-        if (int rc = check_nan_and_restore(b, E, I, b->info_host, b->stream, &rolled)) return rc;
-        if (!rolled && I->host_step % ci == 0 && I->host_step % (int64_t(ci) * 20) == 0)
-          if (int rc = do_store(b, I, E.cur, b->info_host, b->stream)) return rc;
+      // the due solves' flags, in one wait
+      std::decay_t<decltype(E.inst)> due;
+      for (auto* I : E.inst)
+        if (I->host_step % std::max(1, I->prm.check_interval) == 0 || it == nsteps) due.push_back(I);
+      auto* infos = reinterpret_cast<cgdev::StepInfo*>(landing(b->info_host));
+      constexpr size_t kInfos = kLanding / sizeof(cgdev::StepInfo);
+      for (size_t k0 = 0; k0 < due.size(); k0 += kInfos) {
+        const size_t k1 = std::min(due.size(), k0 + kInfos);
+        for (size_t k = k0; k < k1; ++k)
+          HIPCHK(b, hipMemcpyAsync(infos + (k - k0), due[k]->info, sizeof(cgdev::StepInfo), hipMemcpyDeviceToHost,
+                                   b->stream));
+        HIPCHK(b, hipStreamSynchronize(b->stream));
+        for (size_t k = k0; k < k1; ++k) {
+          auto* I = due[k];
+          const int ci = std::max(1, I->prm.check_interval);
+          if (infos[k - k0].nan) {
+            bool rolled = false;
+            if (int rc = check_nan_and_restore(b, E, I, b->info_host, b->stream, &rolled)) return rc;
+            continue;
+          }
+          I->host_step = infos[k - k0].step;
+          if (I->host_step % ci == 0 && I->host_step % (int64_t(ci) * 20) == 0)
+            if (int rc = do_store(b, I, E.cur, b->info_host, b->stream)) return rc;
+        }
       }
     }
     HIPCHK(b, hipStreamSynchronize(b->stream));
@@ -3167,7 +3201,7 @@ int cg_batch_get_state(cg_batch* b, int id, double* rho, double* u, double* rhoE
   return with_engine(b, [&](auto& E) -> int {
     auto* I = find_inst(E, id);
     if (!I) return b->set(CG_EINVAL, "no instance " + std::to_string(id));
-    return get_state(b, I, E.cur, rho, u, rhoE, b->stream);
+    return get_state(b, I, E.cur, b->info_host, rho, u, rhoE, b->stream);
   });
 }
 

@@ -64,6 +64,7 @@ template <class R>
 struct GeomT {
   int ncv, nfa, nef;
   const double *inv_vol, *vol, *sa_to_vol, *dcmag, *dx13, *dx23;
+  const int* ext;  // device cell -> mesh cell (null: the same order)
   // compact pairs (thread per pair)
   const int *plo, *phi;                           // the pair's cells (lo < hi in pair orientation)
   const R *pn0, *pn1, *pn2, *pc0, *pc1, *pc2;     // pair n and c (grouping applied)
@@ -136,7 +137,7 @@ struct WorkT {
   R* bacc;           // [5][ncv] boundary part of the boundary cells' RHS (null without boundary faces)
   StepInfo* info;
   double* partial;   // reduction scratch [nblocks][8]
-  double* diag;      // [8]
+  double* diag;      // [8] sums, [8] a CFL maximum
   // DSM_LOCAL only (null otherwise): the filtered fields [ncv][16] (rho, u, the
   // model tensor smag rho S and rho u u, deviatoric-symmetric storage) and the
   // time-relaxed L:M and M:M [ncv] carried from step to step
@@ -287,9 +288,16 @@ template <class R>
 int launch_props(const Launch<R>& L, int cur, int fields, void* stream);
 // per-cell convective CFL into the work field cfl, or (max_bits not null) only
 // its maximum into *max_bits as the bit pattern of a non-negative double (the
-// caller zeroes it first)
+// caller zeroes it first); own_dt: at the solve's own dt
 template <class R>
-int launch_cfl(const Launch<R>& L, int cur, double dt, void* stream, unsigned long long* max_bits = nullptr);
+int launch_cfl(const Launch<R>& L, int cur, double dt, void* stream, unsigned long long* max_bits = nullptr,
+               bool own_dt = false);
+// a one-instance launch's state (out: rho [ncv], u [ncv][3], rhoE [ncv]) or stage
+// RHS [5][ncv] (out [ncv][5]) in mesh order
+template <class R>
+int launch_pack_state(const Launch<R>& L, int ncv, int cur, double* out, void* stream);
+template <class R>
+int launch_pack_rhs(const Launch<R>& L, int ncv, const double* rhs, double* out, void* stream);
 // the 8 diagnostic sums of every instance; partial / out: device buffers for the
 // block partials and the sums (one instance; null: each instance's own buffers)
 template <class R>

@@ -3193,10 +3193,46 @@ __global__ __launch_bounds__(kBlock) void k_nscbc_init(const Inst<R>* __restrict
   }
 }
 
-// per-cell convective CFL at a given dt
+// The state of a one-instance launch as the host takes it, in mesh order:
+// rho [ncv], u [ncv][3], rhoE [ncv] one after the other, so that it leaves the
+// GPU in one copy of 40 bytes a cell and needs no reordering on the host (96^3:
+// 32 -> 2.1 ms per FP64 read, which took the 64-byte records twice).
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_pack_state(const Inst<R>* __restrict__ I, int cur, double* out) {
+  const Inst<R>& X = I[0];
+  const size_t n = X.g.ncv, c = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (c >= n) return;
+  const size_t e = X.g.ext ? G(X.g.ext)[c] : c;
+  const StateT<R> st = X.st[cur];
+  if constexpr (kMixed<R>) {
+    out[e] = G(st.cons)[c];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) out[n + 3 * e + i] = G(st.cons)[(1 + i) * n + c];
+    out[4 * n + e] = G(st.cons)[4 * n + c];
+  } else {
+    const Light<R> L = load_light(st.light, (int)c);
+    out[e] = L.rho;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) out[n + 3 * e + i] = L.u[i];
+    out[4 * n + e] = G(st.rhoE)[c];
+  }
+}
+
+// A stage RHS [5][ncv] in device order as [ncv][5] in mesh order.
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_pack_rhs(const Inst<R>* __restrict__ I, const double* __restrict__ rhs,
+                                                     double* out) {
+  const size_t n = I[0].g.ncv, c = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (c >= n) return;
+  const size_t e = I[0].g.ext ? G(I[0].g.ext)[c] : c;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) out[5 * e + q] = rhs[q * n + c];
+}
+
+// per-cell convective CFL at a given dt (own_dt: the solve's own)
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_cfl(const Inst<R>* __restrict__ I, const int* __restrict__ bmap, int cur,
-                                                double dt, unsigned long long* max_bits) {
+                                                double dt, int own_dt, unsigned long long* max_bits) {
   int lblk;
   const Inst<R>* Xp = inst_of(I, bmap, lblk);
   if (!Xp) return;
@@ -3227,14 +3263,15 @@ __global__ __launch_bounds__(kBlock) void k_cfl(const Inst<R>* __restrict__ I, c
     cfl += mabs(undA) + area * sos_avg;
   }
   double cd = double(cfl);
+  if (own_dt) dt = G(w.info)->dt;
   cd *= 0.5 * dt * G(g.inv_vol)[c];
   if (!max_bits) {
     G(w.cfl)[c] = cd;
     return;
   }
   // the maximum alone, by the bit pattern of the non-negative value (a NaN
-  // is skipped, as a running max with std::max semantics skips it)
-  if (cd == cd) cfl_max(max_bits, (unsigned long long)__double_as_longlong(cd));
+  // is skipped, as a running max from 0 with std::max semantics skips it)
+  if (cd > 0.0) cfl_max(max_bits, (unsigned long long)__double_as_longlong(cd));
 }
 
 // Diagnostics: fixed-shape block reduction of 8 sums (deterministic order), FP64.
@@ -3322,6 +3359,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_final(const Inst<R>* __restrict
     __syncthreads();
   }
   if (threadIdx.x < 8) diag[threadIdx.x] = sh[threadIdx.x][0];
+  if (threadIdx.x == 8) diag[8] = 0.0;  // the CFL maximum of a k_cfl that follows
 }
 
 // EquilibriumWM::solve_qt (wm/EquilibriumWM.hpp:36-205), FP64 in its operation
@@ -3764,9 +3802,21 @@ int launch_zone_sums(const Launch<R>& L, int cur, int stage, void* stream) {
 }
 
 template <class R>
-int launch_cfl(const Launch<R>& L, int cur, double dt, void* stream, unsigned long long* max_bits) {
+int launch_cfl(const Launch<R>& L, int cur, double dt, void* stream, unsigned long long* max_bits, bool own_dt) {
   hipLaunchKernelGGL(k_cfl<R>, dim3(L.nblk), dim3(kBlock), 0, (hipStream_t)stream, L.I, L.bmap, cur, dt,
-                     max_bits);
+                     own_dt ? 1 : 0, max_bits);
+  return check();
+}
+
+template <class R>
+int launch_pack_state(const Launch<R>& L, int ncv, int cur, double* out, void* stream) {
+  hipLaunchKernelGGL(k_pack_state<R>, dim3(blocks_for(ncv)), dim3(kBlock), 0, (hipStream_t)stream, L.I, cur, out);
+  return check();
+}
+
+template <class R>
+int launch_pack_rhs(const Launch<R>& L, int ncv, const double* rhs, double* out, void* stream) {
+  hipLaunchKernelGGL(k_pack_rhs<R>, dim3(blocks_for(ncv)), dim3(kBlock), 0, (hipStream_t)stream, L.I, rhs, out);
   return check();
 }
 
@@ -3863,7 +3913,9 @@ int launch_fill(float* p, float v, int64_t n, void* stream) {
   template int launch_props<R>(const Launch<R>&, int, int, void*);                                \
   template int launch_begin_step<R>(const Launch<R>&, void*);                                     \
   template int launch_nscbc_init<R>(const Launch<R>&, int, bool, void*);                          \
-  template int launch_cfl<R>(const Launch<R>&, int, double, void*, unsigned long long*);          \
+  template int launch_cfl<R>(const Launch<R>&, int, double, void*, unsigned long long*, bool);    \
+  template int launch_pack_state<R>(const Launch<R>&, int, int, double*, void*);                   \
+  template int launch_pack_rhs<R>(const Launch<R>&, int, const double*, double*, void*);           \
   template int launch_diag<R>(const Launch<R>&, int, void*, double*, double*);                   \
   template int launch_rk_apply<R>(int, const Launch<R>&, int, const double*, void*);               \
   template int launch_layout_geom<R>(int64_t, const int*, const double*, const double*, R* const[6], int64_t, \
