@@ -183,7 +183,7 @@ struct Instance : HostInst {
   cgk::Launch<R> solo_launch() const {
     return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, 4, prm.sgs_model == CG_SGS_SIGMA,
             prm.use_full_gr != 0, prm.sgs_model == CG_SGS_DSM_LOCAL, prm.nsc,
-            scalar_lds<R>(lds, prm.nsc, lay->lds_max), lay->g.nbf > 0, zsum, wm ? lay->g.nbf : 0};
+            scalar_lds<R>(lds, prm.nsc, lay->lds_max), lay->g.nbf > 0, zsum, npblocks > 0, wm ? lay->g.nbf : 0};
   }
   cgdev::Inst<R> record() const {
     cgdev::Inst<R> r{};
@@ -1227,10 +1227,12 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
   if (npb) HIPCHK(s, hipMemcpy(E.pbmap, pbmap.data(), sizeof(int) * npb, hipMemcpyHostToDevice));
   // the LDS variant of the extended pass needs a halo on every instance
   bool any_sigma = false, any_full_gr = false, any_dsm = false, any_bf = false, any_zsum = false;
+  bool all_pairs = true;
   int max_nsc = 0, lds_max = 0, wm_nbf = 0;
   for (auto* I : E.inst) {
     any_bf = any_bf || I->lay->g.nbf > 0;
     any_zsum = any_zsum || I->zsum;
+    all_pairs = all_pairs && I->npblocks > 0;
     if (I->wm) wm_nbf = std::max(wm_nbf, I->lay->g.nbf);
     any_sigma = any_sigma || I->prm.sgs_model == CG_SGS_SIGMA;
     any_full_gr = any_full_gr || I->prm.use_full_gr != 0;
@@ -1245,7 +1247,7 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
   const size_t flux_lds = (all_halo && !E.force_global) ? lds : 0;
   E.L = {E.tab, E.bmap, nb, n, flux_lds, flux_lds && all_shalo ? slds : 0, E.pbmap, npb, E.tile, any_sigma,
          any_full_gr, any_dsm, max_nsc, scalar_lds<R>(flux_lds, max_nsc, lds_max), any_bf, any_zsum,
-         wm_nbf};
+         all_pairs, wm_nbf};
   E.dirty = false;
   return 0;
 }
@@ -1255,9 +1257,8 @@ template <class R>
 int engine_launch_step(Err* s, Engine<R>& E, hipStream_t stream) {
   const cgk::Launch<R>& L = E.L;
   if (L.nblk == 0) return 0;
-  if (const int le = cgk::launch_begin_step(L, stream)) return launch_fail(s, "begin_step", le);
   for (int stage = 1; stage <= 3; ++stage) {
-    if (const int le = cgk::launch_flux(stage, 1, L, E.cur, nullptr, stream)) return launch_fail(s, "flux", le);
+    if (const int le = cgk::launch_flux(stage, 1, L, E.cur, nullptr, stream, stage == 1)) return launch_fail(s, "flux", le);
     E.cur ^= 1;
     if (const int le = cgk::launch_grad(L, E.cur, stream)) return launch_fail(s, "grad", le);
   }

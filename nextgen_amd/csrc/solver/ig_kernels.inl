@@ -493,6 +493,26 @@ __device__ __forceinline__ void write_rhs(double* rhs_out, int ncv, int c, const
   }
 }
 
+// setDt (FlowSolver.hpp:2274-2328) and the step/time bookkeeping of
+// advanceSolution (time += dt, -= dt/2, += dt/2).
+__device__ __forceinline__ void begin_step(StepInfo* s, const Params& P) {
+  #pragma clang fp contract(off)  // FP64: rounded as the reference rounds
+  if (s->nan) return;
+  const double cfl_max = __longlong_as_double((long long)s->cfl_bits);
+  double dt;
+  if (P.dt_mode == 0) dt = P.dt_data0;
+  else if (P.dt_mode == 1) dt = P.dt_data0 / cfl_max;
+  else if (P.dt_mode == 2) dt = smin(P.dt_data1, P.dt_data0 / smax(cfl_max, 1.0E-12));
+  else dt = smin(P.dt_data1 - s->time, P.dt_data0 / smax(cfl_max, 1.0E-12));
+  s->dt = dt;
+  s->step += 1;
+  double t = s->time;
+  t += dt;
+  t -= 0.5 * dt;
+  t += 0.5 * dt;
+  s->time = t;
+}
+
 // A 16-byte piece of a record
 template <class R> struct Piece;
 template <> struct Piece<double> { using T = double __attribute__((ext_vector_type(2))); };
@@ -524,9 +544,12 @@ __device__ __forceinline__ void stage_records(const R* __restrict__ rec, int idx
 // thread's own gather costs a cache-line lookup per lane and 16-byte piece, which
 // took more than half of the pass (96^3: FP64 307 -> 260 us, mixed 148 -> 116;
 // 64^3 mixed 46 -> 37; 32^3 FP64 15.2 -> 12.7). 1.18 GB at 96^3 FP64: 4.5 TB/s.
+// With `begin` (stage 1 of a step) the solve's first thread also takes the step's
+// dt and time (begin_step): the first to read them is the flux pass that follows.
+// A launch of its own took 4.5 us a step (16^3 mixed: 84 -> 79 us a step).
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_cpair(const Inst<R>* __restrict__ I, const int* __restrict__ pbmap,
-                                                  int cur) {
+                                                  int cur, int begin) {
   using V = typename Piece<R>::T;
   constexpr int kL = L_N * (int)sizeof(R) / 16, kA = A_N * (int)sizeof(R) / 16;
   constexpr int kStride = kL + kA + 1;  // odd: no bank conflicts between the lanes' reads
@@ -551,6 +574,7 @@ __global__ __launch_bounds__(kBlock) void k_cpair(const Inst<R>* __restrict__ I,
   const R area = ldnt(g.parea + f), aod = ldnt(g.paod + f);
   __builtin_amdgcn_sched_barrier(0);
   if (G(w.info)->nan) return;
+  if (begin && fl == 0) begin_step(w.info, X.P);
   V* mine = lds + (threadIdx.x - lane) * kStride;
   stage_records<L_N, kStride>(in.light, hi, lane, mine);
   stage_records<A_N, kStride>(w.aux, hi, lane, mine + kL);
@@ -3049,26 +3073,6 @@ __global__ __launch_bounds__(5 * kSlice) void k_props_rows(const Inst<R>* __rest
   props_sensor<R, FIELDS>(g, w, P, c, vv2);
 }
 
-// setDt (FlowSolver.hpp:2274-2328) and the step/time bookkeeping of
-// advanceSolution (time += dt, -= dt/2, += dt/2).
-__device__ __forceinline__ void begin_step(StepInfo* s, const Params& P) {
-  #pragma clang fp contract(off)  // FP64: rounded as the reference rounds
-  if (s->nan) return;
-  const double cfl_max = __longlong_as_double((long long)s->cfl_bits);
-  double dt;
-  if (P.dt_mode == 0) dt = P.dt_data0;
-  else if (P.dt_mode == 1) dt = P.dt_data0 / cfl_max;
-  else if (P.dt_mode == 2) dt = smin(P.dt_data1, P.dt_data0 / smax(cfl_max, 1.0E-12));
-  else dt = smin(P.dt_data1 - s->time, P.dt_data0 / smax(cfl_max, 1.0E-12));
-  s->dt = dt;
-  s->step += 1;
-  double t = s->time;
-  t += dt;
-  t -= 0.5 * dt;
-  t += 0.5 * dt;
-  s->time = t;
-}
-
 template <class R>
 __global__ void k_begin_step(const Inst<R>* __restrict__ I, int ninst) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ninst; i += gridDim.x * blockDim.x)
@@ -3652,15 +3656,20 @@ constexpr int kPipeBlocks = 1024;
 static_assert(kRowsBlocks<float> <= kRowsMaxBlocks && kRowsBlocks<double> <= kRowsMaxBlocks, "slices' halos");
 
 template <class R>
-int launch_flux(int stage, int mode, const Launch<R>& L, int cur, double* rhs_out, void* stream) {
-  if (launch_flux_compact(L, cur, stream)) return -1;
+int launch_flux(int stage, int mode, const Launch<R>& L, int cur, double* rhs_out, void* stream, bool begin) {
+  if (begin && !L.all_pairs) {
+    if (launch_begin_step(L, stream)) return -1;
+    begin = false;
+  }
+  if (launch_flux_compact(L, cur, stream, begin)) return -1;
   return launch_flux_ext(stage, mode, L, cur, rhs_out, stream);
 }
 
 template <class R>
-int launch_flux_compact(const Launch<R>& L, int cur, void* stream) {
+int launch_flux_compact(const Launch<R>& L, int cur, void* stream, bool begin) {
   if (L.npblk == 0) return 0;
-  hipLaunchKernelGGL(k_cpair<R>, dim3(L.npblk), dim3(kBlock), 0, (hipStream_t)stream, L.I, L.pbmap, cur);
+  hipLaunchKernelGGL(k_cpair<R>, dim3(L.npblk), dim3(kBlock), 0, (hipStream_t)stream, L.I, L.pbmap, cur,
+                     begin ? 1 : 0);
   return check();
 }
 
@@ -3903,8 +3912,8 @@ int launch_fill(float* p, float v, int64_t n, void* stream) {
 #endif
 
 #define CGK_INSTANTIATE(R)                                                                         \
-  template int launch_flux<R>(int, int, const Launch<R>&, int, double*, void*);                   \
-  template int launch_flux_compact<R>(const Launch<R>&, int, void*);                              \
+  template int launch_flux<R>(int, int, const Launch<R>&, int, double*, void*, bool);             \
+  template int launch_flux_compact<R>(const Launch<R>&, int, void*, bool);                        \
   template int launch_flux_ext<R>(int, int, const Launch<R>&, int, double*, void*);               \
   template int launch_zone_sums<R>(const Launch<R>&, int, int, void*);                            \
   template int launch_grad<R>(const Launch<R>&, int, void*);                                      \
