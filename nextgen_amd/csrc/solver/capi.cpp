@@ -862,24 +862,23 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
       rc |= upload(s, &tmp, &d_nf, nf);
       rc |= upload(s, &tmp, &d_fw, fw);
       rc |= upload(s, &tmp, &d_xp, xpair);
-      R* x6[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+      R* xs6 = nullptr;
       R* cn[3] = {nullptr, nullptr, nullptr};
       double* cw = nullptr;
-      for (auto& p : x6) rc |= dev_alloc(s, h, &p, (size_t)xs.nslots);
+      rc |= dev_alloc(s, h, &xs6, 6 * (size_t)xs.nslots);
       for (auto& p : cn) rc |= dev_alloc(s, h, &p, (size_t)cs.nslots);
       rc |= dev_alloc(s, h, &cw, (size_t)cs.nslots);
       if (rc) return rc;
       DevLock lk(g_dev_mu);
       hipStream_t st = nullptr;
       HIPCHK(s, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-      const int le = cgk::launch_layout_geom<R>(xs.nslots, d_xp, d_nU, d_cU, x6, cs.nslots, g.cf_pair, d_nf, d_fw, cn,
+      const int le = cgk::launch_layout_geom<R>(xs.nslots, d_xp, d_nU, d_cU, xs6, cs.nslots, g.cf_pair, d_nf, d_fw, cn,
                                                 cw, st);
       const hipError_t se = hipStreamSynchronize(st);
       (void)hipStreamDestroy(st);
       if (le) return launch_fail(s, "layout geometry", le);
       if (se != hipSuccess) return s->set(CG_EHIP, std::string("layout geometry: ") + hipGetErrorString(se));
-      g.xsn0 = x6[0]; g.xsn1 = x6[1]; g.xsn2 = x6[2];
-      g.xsc0 = x6[3]; g.xsc1 = x6[4]; g.xsc2 = x6[5];
+      g.xs = xs6;
       g.cfn0 = cn[0]; g.cfn1 = cn[1]; g.cfn2 = cn[2];
       g.cfw = cw;
     }

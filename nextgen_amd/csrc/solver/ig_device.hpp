@@ -79,7 +79,9 @@ struct GeomT {
   // purely extended half-faces
   const int *xf_ptr, *xf_deg;
   const int* xf_nbr;                              // neighbour | hi-side flag << 31
-  const R *xsn0, *xsn1, *xsn2, *xsc0, *xsc1, *xsc2;
+  // the slots' pair n and c: 6 x 64 values per row of 64 slots (n0 of the 64 slots,
+  // then n1, ... c2), so that a wavefront streams one run of memory
+  const R* xs;
   // per-block halo for LDS staging (null when staging is off): the sorted
   // cells block b's extended half-faces reach are halo_v[halo_ptr[b] .. halo_ptr[b+1]);
   // xf_loc[slot] = halo position of the slot's neighbour | hi-side flag << 15
@@ -324,7 +326,7 @@ int launch_prims(const Launch<R>& L, int inst, int ncv, int cur, double* out, vo
 // layout setup: the per-slot pair geometry (extended n, c; compact n_fa and
 // filter weight) gathered from the per-pair FP64 arrays on the device
 template <class R>
-int launch_layout_geom(int64_t nx, const int* xpair, const double* nU, const double* cU, R* const x6[6], int64_t nc,
+int launch_layout_geom(int64_t nx, const int* xpair, const double* nU, const double* cU, R* xs, int64_t nc,
                        const int* cpair, const double* nfa, const double* fw, R* const cn[3], double* cw,
                        void* stream);
 int launch_fill(double* p, double v, int64_t n, void* stream);

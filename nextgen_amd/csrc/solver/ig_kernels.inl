@@ -221,6 +221,24 @@ __device__ __forceinline__ void flux_symmetric(R cF[5], const R c[3], const R u_
   cF[4] = h_stag * dFrho + Frho * dH;
 }
 
+// Geometry of the slot at row k, lane l of a slice whose extended rows start at
+// slot xp0: its pair's n and c, six rows of 64 values one after the other (one
+// address per row instead of six; against six arrays the pipelined pass of twelve
+// FP64 solves 158 -> 148 us, of 64^3 mixed 125 -> 120; 96^3 is the same).
+template <class R>
+__device__ __forceinline__ const R* ext_rows(const GeomT<R>& g, int xp0) {
+  return g.xs + 6 * (size_t)xp0;
+}
+template <class R>
+__device__ __forceinline__ void ld_geom(R n[3], R cv[3], const R* rows, int k, int l) {
+  const R* q = rows + (6 * kSlice * k + l);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    n[d] = ldnt(q + d * kSlice);
+    cv[d] = ldnt(q + (3 + d) * kSlice);
+  }
+}
+
 // x with its sign flipped when neg (exact: one bit operation)
 __device__ __forceinline__ double flip(double x, bool neg) {
   return __longlong_as_double(__double_as_longlong(x) ^ (long long)((unsigned long long)neg << 63));
@@ -546,7 +564,7 @@ __device__ __forceinline__ void stage_records(const R* __restrict__ rec, int idx
 // 64^3 mixed 46 -> 37; 32^3 FP64 15.2 -> 12.7). 1.18 GB at 96^3 FP64: 4.5 TB/s.
 // With `begin` (stage 1 of a step) the solve's first thread also takes the step's
 // dt and time (begin_step): the first to read them is the flux pass that follows.
-// A launch of its own took 4.5 us a step (16^3 mixed: 84 -> 79 us a step).
+// A launch of its own took 4.5 us on the stream (16^3 mixed: 80 -> 77 us a step).
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_cpair(const Inst<R>* __restrict__ I, const int* __restrict__ pbmap,
                                                   int cur, int begin) {
@@ -1353,14 +1371,15 @@ __global__ __launch_bounds__(kBlock) void k_flux(const Inst<R>* __restrict__ I, 
   R acc[5];
   boundary_flux(g, w, in, P, c, self, acc, STAGE, MODE == 1);
   gather_compact(g, w, pos, acc);
+  const R* const xr = ext_rows(g, G(g.xf_ptr)[pos >> 6]);
   for (int k = 0; k < deg; ++k) {
     const int slot = base + k * kSlice;
     const int code = ldnt(g.xf_nbr + slot);
     const int nb = code & 0x7fffffff;
     const bool self_hi = code < 0;
     const Light<R> other = load_light(in.light, nb);
-    const R n[3] = {ldnt(g.xsn0 + slot), ldnt(g.xsn1 + slot), ldnt(g.xsn2 + slot)};
-    const R cv[3] = {ldnt(g.xsc0 + slot), ldnt(g.xsc1 + slot), ldnt(g.xsc2 + slot)};
+    R n[3], cv[3];
+    ld_geom(n, cv, xr, k, pos & (kSlice - 1));
     add_half_face(acc, n, cv, self, other, self_hi);
   }
 
@@ -1413,6 +1432,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_lds(const Inst<R>* __restrict__
   // slots are fetched NB at a time so their global loads overlap (NB is a
   // tuning choice); the accumulation order stays k = 0, 1, ...
   constexpr int kBatch = NB;
+  const R* const xr = ext_rows(g, G(g.xf_ptr)[pos >> 6]);
   for (int k0 = 0; k0 < deg; k0 += kBatch) {
     int code[kBatch];
     R n[kBatch][3], cv[kBatch][3];
@@ -1421,8 +1441,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_lds(const Inst<R>* __restrict__
       if (k0 + j < deg) {
         const int slot = base + (k0 + j) * kSlice;
         code[j] = ldnt(g.xf_loc + slot);
-        n[j][0] = ldnt(g.xsn0 + slot); n[j][1] = ldnt(g.xsn1 + slot); n[j][2] = ldnt(g.xsn2 + slot);
-        cv[j][0] = ldnt(g.xsc0 + slot); cv[j][1] = ldnt(g.xsc1 + slot); cv[j][2] = ldnt(g.xsc2 + slot);
+        ld_geom(n[j], cv[j], xr, k0 + j, pos & (kSlice - 1));
       }
     }
 #pragma unroll
@@ -1554,14 +1573,14 @@ __global__ __launch_bounds__(kBlock) void k_flux_pipe(const Inst<R>* __restrict_
     R n[3], cv[3];
     int code;
   };
+  const R* const xr = ext_rows(g, xp0);
   auto ld = [&](Row(&r)[kNB], int k0) {
 #pragma unroll
     for (int j = 0; j < kNB; ++j) {
       const int k = k0 + j;
-      const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < deg ? lane : 0);
-      r[j].code = ldnt(g.xf_loc + slot);
-      r[j].n[0] = ldnt(g.xsn0 + slot); r[j].n[1] = ldnt(g.xsn1 + slot); r[j].n[2] = ldnt(g.xsn2 + slot);
-      r[j].cv[0] = ldnt(g.xsc0 + slot); r[j].cv[1] = ldnt(g.xsc1 + slot); r[j].cv[2] = ldnt(g.xsc2 + slot);
+      const int row = k < nrow ? k : nrow - 1, l = k < deg ? lane : 0;
+      r[j].code = ldnt(g.xf_loc + (xp0 + row * kSlice + l));
+      ld_geom(r[j].n, r[j].cv, xr, row, l);
     }
   };
   auto add = [&](const Row(&r)[kNB], int k0) {
@@ -1675,11 +1694,11 @@ __global__ __launch_bounds__(W* kSlice) void k_flux_rows(const Inst<R>* __restri
     R n[3], cv[3];
     int code;
   };
+  const R* const xr = ext_rows(g, xp0);
   auto ld_row = [&](Row& r, int k) {
-    const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < deg ? lane : 0);
-    r.code = ldnt(g.sh_loc + slot);
-    r.n[0] = ldnt(g.xsn0 + slot); r.n[1] = ldnt(g.xsn1 + slot); r.n[2] = ldnt(g.xsn2 + slot);
-    r.cv[0] = ldnt(g.xsc0 + slot); r.cv[1] = ldnt(g.xsc1 + slot); r.cv[2] = ldnt(g.xsc2 + slot);
+    const int row = k < nrow ? k : nrow - 1, l = k < deg ? lane : 0;
+    r.code = ldnt(g.sh_loc + (xp0 + row * kSlice + l));
+    ld_geom(r.n, r.cv, xr, row, l);
   };
   for (int i = threadIdx.x; i < hs; i += W * kSlice) {
     const auto q = G(in.light + (size_t)G(g.sh_v)[hb + i] * L_N);
@@ -1944,15 +1963,15 @@ __global__ __launch_bounds__(kBlock) void k_scalars(const Inst<R>* __restrict__ 
     R n[3], cv[3];
     int code;
   };
+  const R* const xr = ext_rows(g, xp0);
   auto ld = [&](Row(&r)[kB], int k0) {
 #pragma unroll
     for (int j = 0; j < kB; ++j) {
       const int k = k0 + j;
-      const int slot = xp0 + (k < nrow ? k : nrow - 1) * kSlice + (k < deg ? lane : 0);
-      if constexpr (LDS) r[j].code = ldnt(g.xf_loc + slot);
-      else r[j].code = ldnt(g.xf_nbr + slot);
-      r[j].n[0] = ldnt(g.xsn0 + slot); r[j].n[1] = ldnt(g.xsn1 + slot); r[j].n[2] = ldnt(g.xsn2 + slot);
-      r[j].cv[0] = ldnt(g.xsc0 + slot); r[j].cv[1] = ldnt(g.xsc1 + slot); r[j].cv[2] = ldnt(g.xsc2 + slot);
+      const int row = k < nrow ? k : nrow - 1, l = k < deg ? lane : 0;
+      if constexpr (LDS) r[j].code = ldnt(g.xf_loc + (xp0 + row * kSlice + l));
+      else r[j].code = ldnt(g.xf_nbr + (xp0 + row * kSlice + l));
+      ld_geom(r[j].n, r[j].cv, xr, row, l);
     }
   };
   auto add_rows = [&](const Row(&r)[kB], int k0) {
@@ -3857,19 +3876,15 @@ int launch_rk_apply(int stage, const Launch<R>& L, int cur, const double* rhs, v
 // and the test-filter weight of pair cpair[i] & 0x7fffffff (cpair == -1: padding).
 template <class R>
 __global__ void k_layout_geom(int64_t nx, const int* __restrict__ xpair, const double* __restrict__ nU,
-                              const double* __restrict__ cU, R* xn0, R* xn1, R* xn2, R* xc0, R* xc1, R* xc2,
-                              int64_t nc, const int* __restrict__ cpair, const double* __restrict__ nfa,
+                              const double* __restrict__ cU, R* xs, int64_t nc, const int* __restrict__ cpair, const double* __restrict__ nfa,
                               const double* __restrict__ fw, R* cn0, R* cn1, R* cn2, double* cw) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nx) {
     const int p = xpair[i];
-    if (p >= 0) {
-      const size_t b = 3 * (size_t)p;
-      xn0[i] = R(nU[b]); xn1[i] = R(nU[b + 1]); xn2[i] = R(nU[b + 2]);
-      xc0[i] = R(cU[b]); xc1[i] = R(cU[b + 1]); xc2[i] = R(cU[b + 2]);
-    } else {
-      xn0[i] = R(0); xn1[i] = R(0); xn2[i] = R(0);
-      xc0[i] = R(0); xc1[i] = R(0); xc2[i] = R(0);
+    R* q = xs + 6 * (i - i % kSlice) + i % kSlice;
+    for (int d = 0; d < 3; ++d) {
+      q[d * kSlice] = p >= 0 ? R(nU[3 * (size_t)p + d]) : R(0);
+      q[(3 + d) * kSlice] = p >= 0 ? R(cU[3 * (size_t)p + d]) : R(0);
     }
   }
   if (i < nc) {
@@ -3886,13 +3901,13 @@ __global__ void k_layout_geom(int64_t nx, const int* __restrict__ xpair, const d
 }
 
 template <class R>
-int launch_layout_geom(int64_t nx, const int* xpair, const double* nU, const double* cU, R* const x6[6], int64_t nc,
+int launch_layout_geom(int64_t nx, const int* xpair, const double* nU, const double* cU, R* xs, int64_t nc,
                        const int* cpair, const double* nfa, const double* fw, R* const cn[3], double* cw,
                        void* stream) {
   const int64_t n = nx > nc ? nx : nc;
   if (n <= 0) return 0;
   hipLaunchKernelGGL(k_layout_geom<R>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, nx,
-                     xpair, nU, cU, x6[0], x6[1], x6[2], x6[3], x6[4], x6[5], nc, cpair, nfa, fw, cn[0], cn[1], cn[2],
+                     xpair, nU, cU, xs, nc, cpair, nfa, fw, cn[0], cn[1], cn[2],
                      cw);
   return check();
 }
@@ -3927,7 +3942,7 @@ int launch_fill(float* p, float v, int64_t n, void* stream) {
   template int launch_pack_rhs<R>(const Launch<R>&, int, const double*, double*, void*);           \
   template int launch_diag<R>(const Launch<R>&, int, void*, double*, double*);                   \
   template int launch_rk_apply<R>(int, const Launch<R>&, int, const double*, void*);               \
-  template int launch_layout_geom<R>(int64_t, const int*, const double*, const double*, R* const[6], int64_t, \
+  template int launch_layout_geom<R>(int64_t, const int*, const double*, const double*, R*, int64_t, \
                                      const int*, const double*, const double*, R* const[3], double*, void*);
 
 }  // namespace cgk
