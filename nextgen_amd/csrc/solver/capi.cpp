@@ -1031,7 +1031,7 @@ int build_instance(Err* s, Instance<R>* I, std::shared_ptr<Layout<R>> lay, const
     if (lay->g.nbf > 0) rc |= dev_alloc(s, h, &w.mf_bf, (size_t)lay->g.nbf);
   }
   rc |= dev_alloc(s, h, &w.aux, (size_t)ncv * cgdev::A_N);
-  if (!mixed) rc |= dev_alloc(s, h, &w.thermo, 2 * (size_t)ncv);
+  if (!mixed) rc |= dev_alloc(s, h, &w.logp, ncv);
   double** wf[] = {&w.T, &w.mu_lam, &w.mu_sgs, &w.loc_lam, &w.loc_sgs, &w.a_sgs, &w.vv2, &w.cfl};
   for (auto pp : wf) rc |= dev_alloc(s, h, pp, ncv);
   if (p->sgs_model == CG_SGS_DSM_LOCAL) {

@@ -130,7 +130,7 @@ struct StepInfo {
 template <class R>
 struct WorkT {
   R* aux;            // [ncv][16]
-  double* thermo;    // FP64 sensor: [ncv][2] log(p/p_ref), 1/(R T) of the end-of-step state
+  double* logp;      // [ncv] log(p/p_ref) of the end-of-step state (FP64 sensor)
   // per-step fields (diagnostic copies)
   double *T, *mu_lam, *mu_sgs, *loc_lam, *loc_sgs, *a_sgs, *vv2, *cfl;
   R* rhs0;           // [5][ncv]

@@ -438,10 +438,7 @@ __device__ __forceinline__ void rk_update(const Geom& g, const State& in, const 
   const Light<double> L = eos(P, rho, u, rhoE, T);
   store_light(out.light, c, L);
   G(out.rhoE)[c] = rhoE;
-  if (STAGE == 3) {
-    G(w.thermo)[2 * (size_t)c] = log(L.p * P.inv_pref);
-    G(w.thermo)[2 * (size_t)c + 1] = 1.0 / (P.R_gas * T);
-  }
+  if (STAGE == 3) G(w.logp)[c] = log(L.p * P.inv_pref);
 }
 
 // Mixed precision: FP32 registers (energy row gauged), FP64 combination,
@@ -2153,8 +2150,7 @@ __global__ __launch_bounds__(kBlock) void k_eos(const Inst<R>* __restrict__ I, c
     const Light<double> in = load_light(st.light, c);
     const Light<double> L = eos(P, in.rho, in.u, G(st.rhoE)[c], T);
     store_light(st.light, c, L);
-    G(w.thermo)[2 * (size_t)c] = log(L.p * P.inv_pref);
-    G(w.thermo)[2 * (size_t)c + 1] = 1.0 / (P.R_gas * T);
+    G(w.logp)[c] = log(L.p * P.inv_pref);
   }
 }
 
@@ -2684,9 +2680,22 @@ __global__ __launch_bounds__(kBlock) void k_sensor_full(const Inst<R>* __restric
 }
 
 // The properties of one cell from its own state and velocity gradient: SGS
-// coefficients and material properties, written to its aux record (all but fgr).
+// coefficients and material properties, for its aux record (all but fgr).
+template <class R>
+struct CellProps {
+  R mu, loc, a_sgs, symh, symp;
+};
+template <class R>
+__device__ __forceinline__ void store_props(const WorkT<R>& w, int c, const CellProps<R>& v) {
+  const auto a = G(w.aux + (size_t)c * A_N);
+  a[A_MU] = v.mu;
+  a[A_LOC] = v.loc;
+  a[A_ASGS] = v.a_sgs;
+  a[A_SYMH] = v.symh;
+  a[A_SYMP] = v.symp;
+}
 template <class R, int FIELDS>
-__device__ __forceinline__ void props_cell(const GeomT<R>& g, const WorkT<R>& w, const Params& P, int c,
+__device__ __forceinline__ CellProps<R> props_cell(const GeomT<R>& g, const WorkT<R>& w, const Params& P, int c,
                                            const Light<R>& self) {
   const R Rg = R(P.R_gas);
   const R pg = kMixed<R> ? R(P.p_g) : R(0);
@@ -2760,11 +2769,6 @@ __device__ __forceinline__ void props_cell(const GeomT<R>& g, const WorkT<R>& w,
   const R symp = smax(R(P.coeff_p) * R(G(g.dcmag)[c]) * lambda / sos2 - R(G(g.dx23)[c]) * a_sgs, R(0));
   const R symh = R(P.coeff_h) * R(G(g.dcmag)[c]);
 
-  auxc[A_MU] = mu_lam + mu_sgs;
-  auxc[A_LOC] = loc_lam + loc_sgs;
-  auxc[A_ASGS] = a_sgs;
-  auxc[A_SYMH] = symh;
-  auxc[A_SYMP] = symp;
   if (FIELDS) {
     G(w.T)[c] = T;
     G(w.mu_lam)[c] = mu_lam;
@@ -2774,6 +2778,7 @@ __device__ __forceinline__ void props_cell(const GeomT<R>& g, const WorkT<R>& w,
     G(w.a_sgs)[c] = a_sgs;
   }
   if (rho != rho || p != p || T != T) G(w.info)->nan = 1;
+  return {mu_lam + mu_sgs, loc_lam + loc_sgs, a_sgs, symh, symp};
 }
 
 // What a cell's sensor and CFL sums give: fgr from the Gibbs remainder's maximum,
@@ -2795,16 +2800,18 @@ __device__ __forceinline__ double props_cfl(const GeomT<R>& g, int c, R cfl) {
 }
 
 // Per-cell terms of the Gibbs remainder: p, sp_vol, 1/(R T) = 1/(R (p / (rho R)))
-// and ln p (FP64) or 1/p with p absolute (mixed precision). In FP64 the last two
-// are kept per cell (w.thermo, with the state), in mixed precision formed here.
+// and ln p (FP64, kept with the state) or 1/p with p absolute (mixed precision).
+// (1/(R T) kept beside ln p made the FP64 pass 6% slower on 2.1M cells,
+// 0.680 against 0.640 ms: more bytes per gather than the divisions cost.)
 template <class R>
 struct Gibbs {
   R p, spv, irt, l4;
 };
 template <class R>
 __device__ __forceinline__ Gibbs<R> gibbs_of(const WorkT<R>& w, R Rg, R pg, R p, R spv, R rho, int c) {
-  if constexpr (kMixed<R>) return {p, spv, mdiv(R(1), Rg * mdiv(p + pg, rho * Rg)), mdiv(R(1), p + pg)};
-  else return {p, spv, G(w.thermo)[2 * (size_t)c + 1], G(w.thermo)[2 * (size_t)c]};
+  const R irt = mdiv(R(1), Rg * mdiv(kMixed<R> ? p + pg : p, rho * Rg));
+  if constexpr (kMixed<R>) return {p, spv, irt, mdiv(R(1), p + pg)};
+  else return {p, spv, irt, G(w.logp)[c]};
 }
 // |Gibbs remainder| of one pair: with dp = p1 - p0 along the pair,
 //   FP64  ln p1 - ln p0 - v_avg dp beta_avg: every term changes sign exactly with
@@ -2837,7 +2844,7 @@ __device__ __forceinline__ R cfl_term(const R n[3], const Light<R>& self, const 
 
 // Properties pass, thread per cell. In mixed precision it was bound by one CFL
 // atomic per wavefront on one address; with one per block that raises the maximum
-// 96^3 cells take 166 us (233), 64^3 62 us (97). FP64 (289 us, 285) is bound by
+// 96^3 cells take 161 us (233), 64^3 59 us (97). FP64 (274 us, 285) is bound by
 // its gathers: 2.2 GB per 2.1M cells at 3.5 TB/s.
 template <class R, int FIELDS, bool LDS>
 __global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I, const int* __restrict__ bmap,
@@ -2868,7 +2875,8 @@ __global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I,
   if (pos < g.ncv) {
     const int c = cell_at(g.xperm, pos);
     const Light<R> self = load_light(st.light, c);
-    props_cell<R, FIELDS>(g, w, P, c, self);
+    // stored with fgr at the end: a record's line is written once
+    const CellProps<R> cp = props_cell<R, FIELDS>(g, w, P, c, self);
 
     // ---- Gibbs-remainder sensor and convective CFL over the extended half-faces ----
     const int lane = pos & (kSlice - 1), sl = pos >> 6;
@@ -2963,6 +2971,7 @@ __global__ __launch_bounds__(kBlock) void k_props(const Inst<R>* __restrict__ I,
         }
       }
     }
+    store_props(w, c, cp);
     props_sensor<R, FIELDS>(g, w, P, c, vv2);
     cfl_cell = props_cfl(g, c, cfl);
   }
@@ -3059,7 +3068,7 @@ __global__ __launch_bounds__(5 * kSlice) void k_props_rows(const Inst<R>* __rest
   }
   if (ncrow == 0) lds_barrier();  // the halo is staged
   if (wv == W) {
-    if (live) props_cell<R, FIELDS>(g, w, P, c, self);
+    if (live) store_props(w, c, props_cell<R, FIELDS>(g, w, P, c, self));
   } else {
     if (wv == W - 1) {
       const double m = wave_max(live ? props_cfl(g, c, cfl) : 0.0);
