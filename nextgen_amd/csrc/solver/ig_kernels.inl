@@ -595,7 +595,10 @@ __global__ __launch_bounds__(kBlock) void k_cpair(const Inst<R>* __restrict__ I,
   stage_records<A_N, kStride>(w.aux, hi, lane, mine + kL);
   const Light<R> a = load_light(in.light, lo);
   const Aux<R> A0 = load_aux(w.aux, lo);
+  // the pieces written by the wavefront's other lanes
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
   __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
   union {
     V v[kL + kA];
     R r[L_N + A_N];
