@@ -181,7 +181,7 @@ struct Instance : HostInst {
   cgdev::Inst<R>* solo = nullptr;    // one-entry device table of this instance
   int slot = -1;                     // its entry in its engine's device table
   cgk::Launch<R> solo_launch() const {
-    return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, 4, prm.sgs_model == CG_SGS_SIGMA,
+    return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, cgk::kTileBySize, prm.sgs_model == CG_SGS_SIGMA,
             prm.use_full_gr != 0, prm.sgs_model == CG_SGS_DSM_LOCAL, prm.nsc,
             scalar_lds<R>(lds, prm.nsc, lay->lds_max), lay->g.nbf > 0, zsum, npblocks > 0, wm ? lay->g.nbf : 0};
   }
@@ -220,7 +220,7 @@ struct Engine {
   int cur = 0;            // st[cur] holds the current state of every instance
   bool dirty = true;      // table / block map need rebuilding
   bool force_global = false;
-  int tile = 4;           // extended slots per batch in the LDS pass
+  int tile = cgk::kTileBySize;  // extended slots per batch of the plain LDS pass (Launch::tile)
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // two captured steps from parity cur (which they return to)
   // host copies of the device table and block maps; a removed solve leaves
   // its entries empty (-1, nblocks 0) until the next rebuild
@@ -2430,8 +2430,7 @@ int cg_create(const cg_mesh* m, const cg_params* p, cg_solver** out) {
     if (!rc) s->ed.inst.push_back(s->id);
   }
   if (rc) return bail(rc);
-  // CG_TILE: extended slots per batch of the LDS pass (2, 4 or 8; as the
-  // batch option "tile")
+  // CG_TILE: as the batch option "tile"
   int tile = 0;
   if (const char* t = std::getenv("CG_TILE")) tile = std::atoi(t);
   if (tile && tile != 2 && tile != 4 && tile != 8) return bail(s->set(CG_EINVAL, "CG_TILE must be 2, 4 or 8"));
@@ -3255,7 +3254,7 @@ int cg_batch_set_option(cg_batch* b, const char* name, int value) {
 int cg_batch_tune(cg_batch* b, int nsteps, char* report, int64_t report_len) {
   if (!b || nsteps < 2) return fail(CG_EINVAL, "bad argument");
   struct Variant { int lds, tile; double ms; };
-  std::vector<Variant> vs = {{1, 2, 0}, {1, 4, 0}, {1, 8, 0}, {0, 4, 0}};
+  std::vector<Variant> vs = {{1, 2, 0}, {1, cgk::kTileBySize, 0}, {1, 8, 0}, {0, cgk::kTileBySize, 0}};
   const bool graph = b->use_graph;
   b->use_graph = true;
   std::string text;

@@ -253,6 +253,9 @@ namespace cgk {
 // the most cell blocks of a launch that takes the row-split passes: layouts of
 // larger meshes carry no slice halos
 constexpr int kRowsMaxBlocks = 384;
+// the extended slots per batch of the plain LDS flux pass unless set otherwise; set
+// to another value, a launch of any size takes that pass
+constexpr int kTileBySize = 4;
 template <class R>
 struct Launch {
   const cgdev::Inst<R>* I;
@@ -263,7 +266,8 @@ struct Launch {
   size_t slds;       // dynamic LDS bytes of the row-split flux pass (0: not available)
   const int* pbmap;  // compact-pair blocks
   int npblk;
-  int tile;          // extended slots fetched per batch in the LDS pass (2, 4 or 8)
+  int tile;          // kTileBySize: passes by the launch's size; 2 or 8: the plain LDS passes, that many
+                     // extended slots fetched per batch
   int sigma;         // some instance uses SGS_MODEL SIGMA (its SGS pass runs first)
   int full_gr;       // some instance uses USE_FULL_GR (its sensor pass runs first)
   int dsm;           // some instance uses SGS_MODEL DSM_LOCAL (its two passes run first)

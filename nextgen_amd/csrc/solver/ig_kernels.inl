@@ -3665,7 +3665,8 @@ int launch_scalars(int stage, const Launch<R>& L, int cur, hipStream_t s) {
   return launch_scalars_n<R, 8>(stage, L, cur, s);
 }
 
-// Which flux pass a launch of nblk cell blocks takes (all give the same bits).
+// Which flux pass a launch of nblk cell blocks takes (all give the same bits)
+// where its tile leaves the choice to the size.
 // Row-split while every slice's workgroup is resident at once (3 per CU in FP64,
 // 6 in mixed precision: 192 and 384 blocks on 256 CUs); beyond that its halos and
 // barriers cost more than its parallelism gives. Ten wavefronts per slice while
@@ -3685,6 +3686,15 @@ constexpr int kRows10Blocks = 64;
 // wavefronts share in L2 (96^3, 3456 blocks: 740 / 758 us FP64, 400 / 424 mixed).
 constexpr int kPipeBlocks = 1024;
 static_assert(kRowsBlocks<float> <= kRowsMaxBlocks && kRowsBlocks<double> <= kRowsMaxBlocks, "slices' halos");
+
+template <class R>
+bool takes_rows(const Launch<R>& L) {
+  return L.tile == kTileBySize && L.slds && L.nblk <= kRowsBlocks<R>;
+}
+template <class R>
+bool takes_pipe(const Launch<R>& L) {
+  return L.tile == kTileBySize && L.lds && L.nblk <= kPipeBlocks;
+}
 
 template <class R>
 int launch_flux(int stage, int mode, const Launch<R>& L, int cur, double* rhs_out, void* stream, bool begin) {
@@ -3724,7 +3734,7 @@ int launch_flux_ext(int stage, int mode, const Launch<R>& L, int cur, double* rh
     hipLaunchKernelGGL(k_zone_sums<R>, dim3(L.ninst), dim3(kBlock), 0, s, L.I, cur, stage);
     if (int rc = check()) return rc;
   }
-  const bool rows = L.slds && L.nblk <= kRowsBlocks<R>, pipe = L.lds && L.nblk <= kPipeBlocks;
+  const bool rows = takes_rows(L), pipe = takes_pipe(L);
   if (L.boundary && (rows || pipe)) {
     hipLaunchKernelGGL(k_bflux<R>, grid, block, 0, s, L.I, L.bmap, cur, mode == 0 ? 1 : stage, mode);
     if (int rc = check()) return rc;
@@ -3760,7 +3770,7 @@ int launch_flux_ext(int stage, int mode, const Launch<R>& L, int cur, double* rh
     };
     if (L.tile == 2) go(std::integral_constant<int, 2>());
     else if (L.tile == 8) go(std::integral_constant<int, 8>());
-    else go(std::integral_constant<int, 4>());
+    else go(std::integral_constant<int, kTileBySize>());
     return check();
   }
   if (mode == 0) hipLaunchKernelGGL((k_flux<R, 1, 0>), grid, block, 0, s, L.I, L.bmap, cur, rhs_out);
@@ -3806,7 +3816,7 @@ int launch_props(const Launch<R>& L, int cur, int fields, void* stream) {
   // mu_lam) every step
   const size_t lds = L.lds / 6 * 4;
   fields = (fields || L.scalars || L.boundary) ? 1 : 0;
-  if (L.slds && L.nblk <= kRowsBlocks<R>) {
+  if (takes_rows(L)) {
     const dim3 grid(slice_grid(L.nblk)), block(5 * kSlice);
     if (fields) hipLaunchKernelGGL((k_props_rows<R, 1>), grid, block, L.slds / 6 * 4, s, L.I, L.bmap, L.nblk, cur);
     else hipLaunchKernelGGL((k_props_rows<R, 0>), grid, block, L.slds / 6 * 4, s, L.I, L.bmap, L.nblk, cur);
