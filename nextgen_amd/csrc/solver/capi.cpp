@@ -749,8 +749,9 @@ int build_layout(Err* s, Layout<R>* Lay, const cg_mesh* m, bool allow_lds) {
       const int nblk = (ncv + cgdev::kBlock - 1) / cgdev::kBlock;
       std::vector<std::vector<int>> halos(nblk);
       std::vector<int16_t> loc(xs.nslots, 0);
-      // slices' halos: the subsets of their block's that each slice reaches
-      const bool slices = nblk <= cgk::kRowsMaxBlocks;
+      // slices' halos: the subsets of their block's that each slice reaches, where
+      // a launch over this mesh can take the row-split passes
+      const bool slices = allow_lds && nblk <= cgk::kRowsBlocks<R>;
       const int nsl = slices ? (ncv + cgdev::kSlice - 1) / cgdev::kSlice : 0;
       std::vector<std::vector<int>> shalos(nsl);
       std::vector<int16_t> sloc(slices ? xs.nslots : 0, 0);

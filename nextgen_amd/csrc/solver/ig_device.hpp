@@ -250,9 +250,10 @@ constexpr int kBlkBits = 20;  // up to 2^20 blocks (268M cells) per instance, 2^
 // launches, `lds` the dynamic LDS bytes of the extended-face pass (0: the
 // global-gather variant; every instance then needs no halo).
 namespace cgk {
-// the most cell blocks of a launch that takes the row-split passes: layouts of
-// larger meshes carry no slice halos
-constexpr int kRowsMaxBlocks = 384;
+// the most cell blocks of a launch that takes the row-split passes (launch_flux has
+// the figures): layouts of larger meshes carry no slice halos
+template <class R>
+constexpr int kRowsBlocks = sizeof(R) == sizeof(float) ? 384 : 192;
 // the extended slots per batch of the plain LDS flux pass unless set otherwise; set
 // to another value, a launch of any size takes that pass
 constexpr int kTileBySize = 4;

@@ -3676,8 +3676,6 @@ int launch_scalars(int stage, const Launch<R>& L, int cur, hipStream_t s) {
 // 40^3 240 / 223, 44^3 (333) 304 / 295, 56^3 (686) 488 / 500. Five against ten
 // wavefronts: FP64 16^3 158 / 143, 24^3 177 / 163, 28^3 (86) 212 / 217; mixed 24^3
 // 129 / 118, 32^3 154 / 153.
-template <class R>
-constexpr int kRowsBlocks = kMixed<R> ? 384 : 192;
 constexpr int kRows10Blocks = 64;
 // Thread per cell: pipelined loads up to 4 blocks per CU, where the wavefronts are
 // too few to hide a batch's round trip (flux pass, plain / pipelined: twelve solves
@@ -3685,7 +3683,6 @@ constexpr int kRows10Blocks = 64;
 // memory is busy anyway and the deeper queues only evict more of what the
 // wavefronts share in L2 (96^3, 3456 blocks: 740 / 758 us FP64, 400 / 424 mixed).
 constexpr int kPipeBlocks = 1024;
-static_assert(kRowsBlocks<float> <= kRowsMaxBlocks && kRowsBlocks<double> <= kRowsMaxBlocks, "slices' halos");
 
 template <class R>
 bool takes_rows(const Launch<R>& L) {

@@ -50,3 +50,20 @@ def test_size_rules_bitwise(prec, kind, dims, sgs):
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
     assert da.cfl_max == db.cfl_max and da.dt == db.dt
+
+
+# blocks of 256 cells: 188, 193, 250; 381, 389
+@pytest.mark.parametrize("prec,dims,slices", [
+    (CG_PREC_FP64, (37, 36, 36), True), (CG_PREC_FP64, (37, 37, 36), False), (CG_PREC_FP64, (40, 40, 40), False),
+    (CG_PREC_MIXED, (37, 37, 36), True), (CG_PREC_MIXED, (46, 46, 46), True), (CG_PREC_MIXED, (47, 46, 46), False)])
+def test_slice_halos_only_where_read(prec, dims, slices, monkeypatch):
+    # the halos' share of a layout: 2 bytes per extended half-face (a twelfth more for
+    # padding) and 4 bytes per halo cell (about four per cell) for the blocks; as much
+    # again and about 25 bytes a cell for the slices of the row-split passes
+    mesh = Mesh.jittered(dims, 0.3, seed=5)
+    halves = 2 * (mesh.nef - mesh.nfa)
+    with_halos = Layout(mesh, prec)
+    monkeypatch.setenv("CG_NO_LDS", "1")
+    without = Layout(mesh, prec)
+    per_half = (with_halos.bytes() - without.bytes()) / halves
+    assert 2.0 < per_half < 3.0 if not slices else 4.0 < per_half < 6.0
