@@ -1,6 +1,8 @@
 """Which kernels a launch takes: the batch option "tile" (CG_TILE for a solver) at 2
 and 8 runs the plain thread-per-cell LDS passes at every size, at its default the
-passes are chosen by the launch's size. Every choice gives the bits of lds=0.
+passes are chosen by the launch's size. Every choice gives the bits of the global
+gathers (lds=0, CG_NO_LDS): with each boundary type, in each
+layout order, for a step and for a right-hand side alone.
 
 The kernels are read from a trace of the launches, taken in a process of its own so
 that the tracer stays out of the other tests.
@@ -15,7 +17,9 @@ import pytest
 
 from nextgen_amd.batch import Batch
 from nextgen_amd.ic import tgv_params
-from nextgen_amd.ideal_gas import CG_PREC_FP64, CG_PREC_MIXED, Mesh, parse_params
+from nextgen_amd.ideal_gas import CG_PREC_FP64, CG_PREC_MIXED, IdealGasSolver, Mesh, parse_params
+
+from test_gpu_walls import WALLS as BOUNDARIES, channel_state, deck
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +126,69 @@ def test_tile_bitwise(prec, kind, sgs):
     for run in runs[1:]:
         for x, y in zip(run, runs[0]):
             np.testing.assert_array_equal(x, y)
+
+
+def solve(monkeypatch, mesh, text, env, nsteps=3):
+    """State, right-hand side, scalars, dt and CFL maximum after nsteps, under env."""
+    for k in ("CG_NO_LDS", "CG_TILE", "CG_LANE_ORDER", "CG_CELL_ORDER"):
+        monkeypatch.delenv(k, raising=False)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    x = mesh.get("x_cv")
+    s = IdealGasSolver(mesh, parse_params(text))
+    s.set_state(*(channel_state(mesh) if mesh.nbf else mesh.ic_tgv(0.1, 1.4)))
+    for i, name in enumerate(n for n in s.scalar_names() if n != "RES_TIME"):
+        s.set_scalar(name, 0.5 + 0.5 * np.sin((i + 1) * x[:, 0] + x[:, 2]) * np.cos(x[:, 1]))
+    s.init_complete()
+    s.advance_solution(nsteps)
+    d = s.report()
+    out = [*s.get_state(), s.calc_rhs(1), *(s.get_scalar(n) for n in s.scalar_names()), np.array([d.dt, d.cfl_max])]
+    s.close()
+    assert all(np.isfinite(v).all() for v in out)
+    return out
+
+
+def assert_same(monkeypatch, mesh, text, envs):
+    ref = solve(monkeypatch, mesh, text, {"CG_NO_LDS": "1"})
+    for env in envs:
+        got = solve(monkeypatch, mesh, text, env)
+        assert len(got) == len(ref)
+        for a, b in zip(got, ref):
+            np.testing.assert_array_equal(a, b, err_msg=str(env))
+
+
+# the row-split passes and the plain one
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("walls", sorted(BOUNDARIES))
+def test_boundary_types_bitwise(walls, prec, monkeypatch):
+    mesh = Mesh.channel((13, 11, 10), jitter=0.3, seed=7)
+    assert_same(monkeypatch, mesh, deck(BOUNDARIES[walls], prec=prec), [{}, {"CG_TILE": "2"}, {"CG_TILE": "8"}])
+
+
+# the pipelined pass: 208 blocks in FP64, 389 in mixed precision
+@pytest.mark.parametrize("prec,dims", [("FP64", (40, 38, 35)), ("MIXED", (48, 46, 45))])
+@pytest.mark.parametrize("walls", ["cbc_upt+sponge", "nscbc_mt_t0+nscbc", "wmeqiso+wmeqiso"])
+def test_boundary_types_pipelined_bitwise(walls, prec, dims, monkeypatch):
+    mesh = Mesh.channel(dims, jitter=0.3, seed=7)
+    assert_same(monkeypatch, mesh, deck(BOUNDARIES[walls], prec=prec), [{}])
+
+
+# beyond the pipelined pass: 1040 blocks
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+def test_large_channel_bitwise(prec, monkeypatch):
+    mesh = Mesh.channel((65, 64, 64), jitter=0.3, seed=7)
+    assert_same(monkeypatch, mesh, deck(BOUNDARIES["cbc_upt+nscbc"], prec=prec), [{}, {"CG_TILE": "8"}])
+
+
+# layouts in which a slice's first lane need not have the most half-faces: rows past a
+# lane's last read a slot that may be padding
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("dims,sgs,count", [((12, 11, 10), "DSM_LOCAL", 3), ((47, 46, 46), "DSM_LOCAL", 1),
+                                            ((66, 64, 63), "SIGMA", 0)])
+def test_layout_orders_every_pass_bitwise(dims, sgs, count, prec, monkeypatch):
+    mesh = Mesh.jittered(dims, 0.3, seed=11)
+    text = tgv_params(sgs=sgs) + f"PRECISION {prec}\n" + "".join(f"REGISTER_SCALAR Z{i}\n" for i in range(count))
+    orders = [{"CG_LANE_ORDER": "plain"}, {"CG_CELL_ORDER": "sorted256", "CG_LANE_ORDER": "plain"},
+              {"CG_CELL_ORDER": "sorted64"}]
+    orders = orders if dims[0] < 40 else orders[:2]
+    assert_same(monkeypatch, mesh, text, orders + [{**o, "CG_TILE": "2"} for o in orders if dims[0] < 40])

@@ -10,6 +10,8 @@ from nextgen_amd.batch import Batch, Instance, Layout
 from nextgen_amd.ic import tgv_params
 from nextgen_amd.ideal_gas import CG_PREC_FP64, CG_PREC_MIXED, Mesh, parse_params
 
+from test_gpu_flux_passes import assert_same
+
 pytestmark = pytest.mark.gpu
 
 WALLS = ("y0 CBC_UPT 0.1 0.4 0 71.42857142857143 1.0\ny1 NSCBC_OUTLET_P 71.07 0.3 6.28\n")
@@ -67,3 +69,27 @@ def test_slice_halos_only_where_read(prec, dims, slices, monkeypatch):
     without = Layout(mesh, prec)
     per_half = (with_halos.bytes() - without.bytes()) / halves
     assert 2.0 < per_half < 3.0 if not slices else 4.0 < per_half < 6.0
+
+
+# the scalar pass is compiled for 1, 2, 4 and 8 scalars: the counts that fill each and
+# those that leave some unused, and a source (RES_TIME, by name the last here)
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("kind,dims,count,res_time", [
+    ("jittered", (9, 8, 8), 1, False), ("jittered", (9, 8, 8), 2, False), ("jittered", (17, 16, 15), 2, True),
+    ("jittered", (13, 11, 10), 4, False), ("jittered", (13, 11, 10), 4, True), ("jittered", (17, 16, 15), 8, False),
+    ("jittered", (12, 11, 9), 7, True), ("channel", (13, 11, 10), 2, False), ("channel", (13, 11, 10), 6, False),
+    ("lattice", (11, 10, 9), 3, False), ("jittered", (30, 28, 21), 3, False),
+    ("jittered", (40, 38, 36), 2, False), ("jittered", (66, 64, 63), 5, False)])
+def test_scalar_counts_bitwise(kind, dims, count, res_time, prec, monkeypatch):
+    if kind == "lattice":
+        mesh = Mesh.lattice(dims)
+    elif kind == "channel":
+        mesh = Mesh.channel(dims, jitter=0.3, seed=9)
+    else:
+        mesh = Mesh.jittered(dims, 0.3, seed=9)
+    text = tgv_params(sgs="VREMAN") + f"PRECISION {prec}\n" + "".join(f"REGISTER_SCALAR A{i}\n" for i in range(count))
+    text += "RES_TIME\n" if res_time else ""
+    if kind == "channel":
+        inflow = "".join(f" A{i} {0.1 * (i + 1)}" for i in range(count))
+        text += f"y0 CBC_UPT 0.1 0.4 0 71.42857142857143 1.0{inflow}\ny1 NSCBC_OUTLET_P 71.07 0.3 6.28\n"
+    assert_same(monkeypatch, mesh, text, [{}, {"CG_TILE": "2"}])
