@@ -253,7 +253,7 @@ namespace cgk {
 // the most cell blocks of a launch that takes the row-split passes (launch_flux has
 // the figures): layouts of larger meshes carry no slice halos
 template <class R>
-constexpr int kRowsBlocks = sizeof(R) == sizeof(float) ? 384 : 192;
+constexpr int kRowsBlocks = sizeof(R) == sizeof(float) ? 320 : 128;
 // the extended slots per batch of the plain LDS flux pass unless set otherwise; set
 // to another value, a launch of any size takes that pass
 constexpr int kTileBySize = 4;

@@ -3665,23 +3665,29 @@ int launch_scalars(int stage, const Launch<R>& L, int cur, hipStream_t s) {
   return launch_scalars_n<R, 8>(stage, L, cur, s);
 }
 
-// Which flux pass a launch of nblk cell blocks takes (all give the same bits)
-// where its tile leaves the choice to the size.
-// Row-split while every slice's workgroup is resident at once (3 per CU in FP64,
-// 6 in mixed precision: 192 and 384 blocks on 256 CUs); beyond that its halos and
-// barriers cost more than its parallelism gives. Ten wavefronts per slice while
-// there is at most one slice per CU. Measured us/step, thread per cell (pipelined)
-// against row-split, jittered boxes: FP64 24^3 (54 blocks) 272 / 162, 32^3 (128)
-// 276 / 230, 36^3 (183) 307 / 311, 40^3 (250) 341 / 418; mixed 32^3 198 / 154,
-// 40^3 240 / 223, 44^3 (333) 304 / 295, 56^3 (686) 488 / 500. Five against ten
-// wavefronts: FP64 16^3 158 / 143, 24^3 177 / 163, 28^3 (86) 212 / 217; mixed 24^3
-// 129 / 118, 32^3 154 / 153.
+// Which flux pass (and which properties pass with it) a launch of nblk cell blocks
+// takes, all giving the same bits, where its tile leaves the choice to the size.
+// Thresholds measured on this device's 256 CUs; us/step, properties included, of
+// jittered boxes, a jittered channel (c) and the uniform lattice (l).
+// Row-split up to kRowsBlocks: 2 slices per CU in FP64 (128 blocks), 5 in mixed
+// precision (320). Beyond that a slice's halo and barriers cost more than its
+// parallelism gives. Thread per cell (pipelined) against row-split: FP64 16^3 205 /
+// 114, 24^3 (54 blocks) 222 / 132, 32^3 (128) 246 / 201, c 276 / 229, l 102 / 102;
+// 33^3 (141) 260 / 267, c 291 / 292; 36^3 (183) 274 / 290, c 300 / 318, l 119 / 151.
+// Mixed 16^3 149 / 77, 32^3 179 / 129, l 76 / 77, 40^3 (250) 212 / 190, l 92 / 93, 43^3
+// (311) 267 / 234, c 295 / 262; 44^3 (333) 268 / 267, l 114 / 125; 46^3 (381) 284 / 288,
+// c 310 / 316, l 122 / 136.
+// Ten wavefronts per slice while there is at most one slice per CU (five / ten: FP64
+// 24^3 149 / 132, 26^3 (69 blocks) 181 / 184, l 87 / 94; mixed 24^3 106 / 94, 26^3 116 /
+// 111, 40^3 190 / 203).
 constexpr int kRows10Blocks = 64;
 // Thread per cell: pipelined loads up to 4 blocks per CU, where the wavefronts are
-// too few to hide a batch's round trip (flux pass, plain / pipelined: twelve solves
-// of 590 blocks 179 / 158 us FP64, 64^3 mixed 138 / 125 us). On larger launches
-// memory is busy anyway and the deeper queues only evict more of what the
-// wavefronts share in L2 (96^3, 3456 blocks: 740 / 758 us FP64, 400 / 424 mixed).
+// too few to hide a batch's round trip (plain / pipelined: FP64 48^3 (432) 512 / 500,
+// 56^3 (686) 788 / 757, 63^3 (977) 1032 / 1027; mixed 48^3 315 / 295, 56^3 438 / 433,
+// 64^3 650 / 602). On larger launches memory is busy anyway and the deeper queues only
+// evict more of what the wavefronts share in L2 (72^3, 1458 blocks: 1501 / 1509 FP64,
+// 837 / 878 mixed; 96^3, 3456: 3764 / 3811 and 1965 / 2049; just above the limit, 66^3,
+// 1124 blocks, the pipelined pass is still ahead: 1410 / 1268 and 703 / 697).
 constexpr int kPipeBlocks = 1024;
 
 template <class R>

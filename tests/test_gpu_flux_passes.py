@@ -70,11 +70,11 @@ ROUTES = [
     ((12, 12, 12), CG_PREC_FP64, 2, L, 2, "k_props"), ((12, 12, 12), CG_PREC_FP64, 8, L, 8, "k_props"),
     ((12, 12, 12), CG_PREC_MIXED, 2, L, 2, "k_props"), ((12, 12, 12), CG_PREC_MIXED, 8, L, 8, "k_props"),
     ((40, 40, 40), CG_PREC_FP64, 8, L, 8, "k_props"), ((48, 48, 48), CG_PREC_MIXED, 2, L, 2, "k_props"),
-    # the limits of the row-split passes (192 blocks of 256 cells in FP64, 384 in mixed
+    # the limits of the row-split passes (128 blocks of 256 cells in FP64, 320 in mixed
     # precision; ten wavefronts up to 64) and of the pipelined one (1024)
     ((32, 32, 16), CG_PREC_FP64, 4, R, 10, "k_props_rows"), ((33, 32, 16), CG_PREC_FP64, 4, R, 5, "k_props_rows"),
-    ((48, 32, 32), CG_PREC_FP64, 4, R, 5, "k_props_rows"), ((49, 32, 32), CG_PREC_FP64, 4, P, None, "k_props"),
-    ((64, 48, 32), CG_PREC_MIXED, 4, R, 5, "k_props_rows"), ((65, 48, 32), CG_PREC_MIXED, 4, P, None, "k_props"),
+    ((32, 32, 32), CG_PREC_FP64, 4, R, 5, "k_props_rows"), ((33, 32, 32), CG_PREC_FP64, 4, P, None, "k_props"),
+    ((64, 40, 32), CG_PREC_MIXED, 4, R, 5, "k_props_rows"), ((65, 40, 32), CG_PREC_MIXED, 4, P, None, "k_props"),
     ((64, 64, 64), CG_PREC_FP64, 4, P, None, "k_props"), ((65, 64, 64), CG_PREC_FP64, 4, L, 4, "k_props"),
     ((64, 64, 64), CG_PREC_MIXED, 4, P, None, "k_props"), ((65, 64, 64), CG_PREC_MIXED, 4, L, 4, "k_props"),
 ]

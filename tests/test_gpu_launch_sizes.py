@@ -54,10 +54,10 @@ def test_size_rules_bitwise(prec, kind, dims, sgs):
     assert da.cfl_max == db.cfl_max and da.dt == db.dt
 
 
-# blocks of 256 cells: 188, 193, 250; 381, 389
+# blocks of 256 cells: 128, 132, 250; 250, 311, 326
 @pytest.mark.parametrize("prec,dims,slices", [
-    (CG_PREC_FP64, (37, 36, 36), True), (CG_PREC_FP64, (37, 37, 36), False), (CG_PREC_FP64, (40, 40, 40), False),
-    (CG_PREC_MIXED, (37, 37, 36), True), (CG_PREC_MIXED, (46, 46, 46), True), (CG_PREC_MIXED, (47, 46, 46), False)])
+    (CG_PREC_FP64, (32, 32, 32), True), (CG_PREC_FP64, (33, 32, 32), False), (CG_PREC_FP64, (40, 40, 40), False),
+    (CG_PREC_MIXED, (40, 40, 40), True), (CG_PREC_MIXED, (43, 43, 43), True), (CG_PREC_MIXED, (44, 43, 44), False)])
 def test_slice_halos_only_where_read(prec, dims, slices, monkeypatch):
     # the halos' share of a layout: 2 bytes per extended half-face (a twelfth more for
     # padding) and 4 bytes per halo cell (about four per cell) for the blocks; as much
@@ -69,6 +69,16 @@ def test_slice_halos_only_where_read(prec, dims, slices, monkeypatch):
     without = Layout(mesh, prec)
     per_half = (with_halos.bytes() - without.bytes()) / halves
     assert 2.0 < per_half < 3.0 if not slices else 4.0 < per_half < 6.0
+
+
+# the blocks around the row-split passes' limits: 128 and 132, 311 and 326
+@pytest.mark.parametrize("kind", ["jittered", "lattice", "channel"])
+@pytest.mark.parametrize("prec,dims", [("FP64", (32, 32, 32)), ("FP64", (33, 32, 32)), ("MIXED", (43, 43, 43)),
+                                       ("MIXED", (44, 43, 44))])
+def test_row_split_limit_bitwise(prec, dims, kind, monkeypatch):
+    mesh = Mesh.lattice(dims) if kind == "lattice" else getattr(Mesh, kind)(dims, 0.3, 5)
+    text = tgv_params(sgs="VREMAN") + f"PRECISION {prec}\n" + (WALLS if kind == "channel" else "")
+    assert_same(monkeypatch, mesh, text, [{}])
 
 
 # the scalar pass is compiled for 1, 2, 4 and 8 scalars: the counts that fill each and
