@@ -224,18 +224,19 @@ __device__ __forceinline__ void flux_symmetric(R cF[5], const R c[3], const R u_
 // Geometry of the slot at row k, lane l of a slice whose extended rows start at
 // slot xp0: its pair's n and c, six rows of 64 values one after the other (one
 // address per row instead of six; against six arrays the pipelined pass of twelve
-// FP64 solves 158 -> 148 us, of 64^3 mixed 125 -> 120; 96^3 is the same).
+// FP64 solves 158 -> 148 us, of 64^3 mixed 125 -> 120; 96^3 is the same). NT: not
+// kept in the caches.
 template <class R>
 __device__ __forceinline__ const R* ext_rows(const GeomT<R>& g, int xp0) {
   return g.xs + 6 * (size_t)xp0;
 }
-template <class R>
+template <bool NT = true, class R>
 __device__ __forceinline__ void ld_geom(R n[3], R cv[3], const R* rows, int k, int l) {
   const R* q = rows + (6 * kSlice * k + l);
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    n[d] = ldnt(q + d * kSlice);
-    cv[d] = ldnt(q + (3 + d) * kSlice);
+    n[d] = NT ? ldnt(q + d * kSlice) : G(q)[d * kSlice];
+    cv[d] = NT ? ldnt(q + (3 + d) * kSlice) : G(q)[(3 + d) * kSlice];
   }
 }
 
@@ -1954,7 +1955,11 @@ __global__ __launch_bounds__(kBlock) void k_scalars(const Inst<R>* __restrict__ 
     }
   }
   // purely extended pairs, pair order: F_rho as the flux pass computes it; kB rows
-  // at a time, the next kB in flight meanwhile
+  // at a time, the next kB in flight meanwhile. The global variant's rows are kept in
+  // L2 (no non-temporal loads): the next stage's global flux pass finds them there
+  // while they fit (24^3 mixed, that pass 93 -> 61 us, a step with 3 scalars 569 -> 466
+  // us; FP64 695 -> 607; 64^3 mixed 1896 -> 1850, FP64 2565 -> 2607). The halo variant
+  // loses by it (64^3, 4 scalars: FP64 1788 -> 1923, mixed 1101 -> 1124).
   const Light<R> self = load_light(in.light, c);
   const int deg = G(g.xf_deg)[pos];
   const int xp0 = G(g.xf_ptr)[sl], nrow = (G(g.xf_ptr)[sl + 1] - xp0) / kSlice;
@@ -1969,9 +1974,10 @@ __global__ __launch_bounds__(kBlock) void k_scalars(const Inst<R>* __restrict__ 
     for (int j = 0; j < kB; ++j) {
       const int k = k0 + j;
       const int row = k < nrow ? k : nrow - 1, l = k < deg ? lane : 0;
-      if constexpr (LDS) r[j].code = ldnt(g.xf_loc + (xp0 + row * kSlice + l));
-      else r[j].code = ldnt(g.xf_nbr + (xp0 + row * kSlice + l));
-      ld_geom(r[j].n, r[j].cv, xr, row, l);
+      const int slot = xp0 + row * kSlice + l;
+      if constexpr (LDS) r[j].code = ldnt(g.xf_loc + slot);
+      else r[j].code = G(g.xf_nbr)[slot];
+      ld_geom<LDS>(r[j].n, r[j].cv, xr, row, l);
     }
   };
   auto add_rows = [&](const Row(&r)[kB], int k0) {
