@@ -512,8 +512,10 @@ int cg_batch_counts(cg_batch* b, int64_t counts[4]);
  * size: row-split, pipelined, or beyond 1024 blocks of 256 cells the plain one with 4.
  * Every setting gives bit-identical results. */
 int cg_batch_set_option(cg_batch* b, const char* name, int value);
-/* Autotuner: time nsteps steps of the batch under each variant (LDS halos
- * with tile 2, 4, 8; global-gather pass) and keep the fastest. The tuning steps
+/* Autotuner: time nsteps steps of the batch under each variant (LDS halos with
+ * tile 2, 4, 8; global-gather pass) and keep the fastest, the passes with halos
+ * being those of the launch's size: up to 1024 blocks they do not read the tile,
+ * which is left as it was there. The tuning steps
  * are ordinary steps (the instances advance). A text table of the timings and
  * the choice is written to report (report_len bytes, NUL-terminated). */
 int cg_batch_tune(cg_batch* b, int nsteps, char* report, int64_t report_len);

@@ -181,7 +181,7 @@ struct Instance : HostInst {
   cgdev::Inst<R>* solo = nullptr;    // one-entry device table of this instance
   int slot = -1;                     // its entry in its engine's device table
   cgk::Launch<R> solo_launch() const {
-    return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, cgk::kTileBySize, prm.sgs_model == CG_SGS_SIGMA,
+    return {solo, lay->solo_bmap, nblocks, 1, lds, lds ? lay->slds : 0, lay->solo_pbmap, npblocks, cgk::kTile, 0, prm.sgs_model == CG_SGS_SIGMA,
             prm.use_full_gr != 0, prm.sgs_model == CG_SGS_DSM_LOCAL, prm.nsc,
             scalar_lds<R>(lds, prm.nsc, lay->lds_max), lay->g.nbf > 0, zsum, npblocks > 0, wm ? lay->g.nbf : 0};
   }
@@ -220,7 +220,8 @@ struct Engine {
   int cur = 0;            // st[cur] holds the current state of every instance
   bool dirty = true;      // table / block map need rebuilding
   bool force_global = false;
-  int tile = cgk::kTileBySize;  // extended slots per batch of the plain LDS pass (Launch::tile)
+  int tile = cgk::kTile;  // extended slots per batch of the plain LDS pass
+  bool plain = false;     // that pass at every size (a tile other than the default was asked for)
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // two captured steps from parity cur (which they return to)
   // host copies of the device table and block maps; a removed solve leaves
   // its entries empty (-1, nblocks 0) until the next rebuild
@@ -1245,7 +1246,7 @@ int engine_sync(Err* s, Engine<R>& E, hipStream_t stream) {
   E.h_pbmap = pbmap;
   E.hole_blocks = 0;
   const size_t flux_lds = (all_halo && !E.force_global) ? lds : 0;
-  E.L = {E.tab, E.bmap, nb, n, flux_lds, flux_lds && all_shalo ? slds : 0, E.pbmap, npb, E.tile, any_sigma,
+  E.L = {E.tab, E.bmap, nb, n, flux_lds, flux_lds && all_shalo ? slds : 0, E.pbmap, npb, E.tile, E.plain, any_sigma,
          any_full_gr, any_dsm, max_nsc, scalar_lds<R>(flux_lds, max_nsc, lds_max), any_bf, any_zsum,
          all_pairs, wm_nbf};
   E.dirty = false;
@@ -2437,7 +2438,10 @@ int cg_create(const cg_mesh* m, const cg_params* p, cg_solver** out) {
   if (tile && tile != 2 && tile != 4 && tile != 8) return bail(s->set(CG_EINVAL, "CG_TILE must be 2, 4 or 8"));
   rc = with_inst(s, [&](auto& E, auto* I) {
     (void)I;
-    if (tile) E.tile = tile;
+    if (tile) {
+      E.tile = tile;
+      E.plain = tile != cgk::kTile;
+    }
     return engine_sync(s, E, s->stream);
   });
   if (rc) return bail(rc);
@@ -3245,6 +3249,7 @@ int cg_batch_set_option(cg_batch* b, const char* name, int value) {
     if (value != 2 && value != 4 && value != 8) return b->set(CG_EINVAL, "tile must be 2, 4 or 8");
     return with_engine(b, [&](auto& E) -> int {
       E.tile = value;
+      E.plain = value != cgk::kTile;
       E.dirty = true;
       return 0;
     });
@@ -3255,25 +3260,47 @@ int cg_batch_set_option(cg_batch* b, const char* name, int value) {
 int cg_batch_tune(cg_batch* b, int nsteps, char* report, int64_t report_len) {
   if (!b || nsteps < 2) return fail(CG_EINVAL, "bad argument");
   struct Variant { int lds, tile; double ms; };
-  std::vector<Variant> vs = {{1, 2, 0}, {1, cgk::kTileBySize, 0}, {1, 8, 0}, {0, cgk::kTileBySize, 0}};
+  std::vector<Variant> vs = {{1, 2, 0}, {1, cgk::kTile, 0}, {1, 8, 0}, {0, cgk::kTile, 0}};
   const bool graph = b->use_graph;
   b->use_graph = true;
+  // the tile of the plain LDS pass, the choice of the passes left to the size
+  auto set_tile = [&](int tile) {
+    return with_engine(b, [&](auto& E) {
+      E.tile = tile;
+      E.plain = false;
+      E.dirty = true;
+      return 0;
+    });
+  };
+  int had_tile = cgk::kTile;
+  bool reads_tile = false;  // the launch is of the size of the plain LDS pass
+  if (int rc = with_engine(b, [&](auto& E) {
+        had_tile = E.tile;
+        return 0;
+      }))
+    return rc;
   std::string text;
   for (auto& v : vs) {
     if (int rc = cg_batch_set_option(b, "lds", v.lds)) return rc;
-    if (int rc = cg_batch_set_option(b, "tile", v.tile)) return rc;
+    if (int rc = set_tile(v.tile)) return rc;
     // a variant that cannot use LDS (an instance without a halo) runs the global pass
     if (int rc = cg_batch_time_steps(b, nsteps, &v.ms)) return rc;
+    if (int rc = with_engine(b, [&](auto& E) {
+          reads_tile = reads_tile || (E.L.lds && E.L.nblk > cgk::kPipeBlocks);
+          return 0;
+        }))
+      return rc;
     text += "lds " + std::to_string(v.lds) + " tile " + std::to_string(v.tile) + ": " +
             std::to_string(v.ms / nsteps) + " ms/step\n";
   }
-  const Variant* best = &vs[0];
+  Variant best = vs[0];
   for (const auto& v : vs)
-    if (v.ms < best->ms) best = &v;
+    if (v.ms < best.ms) best = v;
+  if (!reads_tile) best.tile = had_tile;  // the same program under every tile
   b->use_graph = graph;
-  if (int rc = cg_batch_set_option(b, "lds", best->lds)) return rc;
-  if (int rc = cg_batch_set_option(b, "tile", best->tile)) return rc;
-  text += "chosen: lds " + std::to_string(best->lds) + " tile " + std::to_string(best->tile) + "\n";
+  if (int rc = cg_batch_set_option(b, "lds", best.lds)) return rc;
+  if (int rc = set_tile(best.tile)) return rc;
+  text += "chosen: lds " + std::to_string(best.lds) + " tile " + std::to_string(best.tile) + "\n";
   if (report && report_len > 0) {
     std::strncpy(report, text.c_str(), (size_t)report_len - 1);
     report[report_len - 1] = '\0';

@@ -254,9 +254,11 @@ namespace cgk {
 // the figures): layouts of larger meshes carry no slice halos
 template <class R>
 constexpr int kRowsBlocks = sizeof(R) == sizeof(float) ? 320 : 128;
-// the extended slots per batch of the plain LDS flux pass unless set otherwise; set
-// to another value, a launch of any size takes that pass
-constexpr int kTileBySize = 4;
+// Thread per cell: the most cell blocks of a launch of the pipelined flux pass
+// (launch_flux has the figures of both limits)
+constexpr int kPipeBlocks = 1024;
+// the extended slots per batch of the plain LDS flux pass unless set otherwise
+constexpr int kTile = 4;
 template <class R>
 struct Launch {
   const cgdev::Inst<R>* I;
@@ -267,8 +269,8 @@ struct Launch {
   size_t slds;       // dynamic LDS bytes of the row-split flux pass (0: not available)
   const int* pbmap;  // compact-pair blocks
   int npblk;
-  int tile;          // kTileBySize: passes by the launch's size; 2 or 8: the plain LDS passes, that many
-                     // extended slots fetched per batch
+  int tile;          // extended slots fetched per batch in the plain LDS flux pass (2, 4 or 8)
+  int plain;         // the plain LDS passes at every size (else by the launch's size)
   int sigma;         // some instance uses SGS_MODEL SIGMA (its SGS pass runs first)
   int full_gr;       // some instance uses USE_FULL_GR (its sensor pass runs first)
   int dsm;           // some instance uses SGS_MODEL DSM_LOCAL (its two passes run first)

@@ -3672,7 +3672,7 @@ int launch_scalars(int stage, const Launch<R>& L, int cur, hipStream_t s) {
 }
 
 // Which flux pass (and which properties pass with it) a launch of nblk cell blocks
-// takes, all giving the same bits, where its tile leaves the choice to the size.
+// takes, all giving the same bits, unless the plain passes are asked for.
 // Thresholds measured on this device's 256 CUs; us/step, properties included, of
 // jittered boxes, a jittered channel (c) and the uniform lattice (l).
 // Row-split up to kRowsBlocks: 2 slices per CU in FP64 (128 blocks), 5 in mixed
@@ -3687,22 +3687,20 @@ int launch_scalars(int stage, const Launch<R>& L, int cur, hipStream_t s) {
 // 24^3 149 / 132, 26^3 (69 blocks) 181 / 184, l 87 / 94; mixed 24^3 106 / 94, 26^3 116 /
 // 111, 40^3 190 / 203).
 constexpr int kRows10Blocks = 64;
-// Thread per cell: pipelined loads up to 4 blocks per CU, where the wavefronts are
+// Thread per cell: pipelined loads up to kPipeBlocks, 4 blocks per CU, where the wavefronts are
 // too few to hide a batch's round trip (plain / pipelined: FP64 48^3 (432) 512 / 500,
 // 56^3 (686) 788 / 757, 63^3 (977) 1032 / 1027; mixed 48^3 315 / 295, 56^3 438 / 433,
 // 64^3 650 / 602). On larger launches memory is busy anyway and the deeper queues only
 // evict more of what the wavefronts share in L2 (72^3, 1458 blocks: 1501 / 1509 FP64,
 // 837 / 878 mixed; 96^3, 3456: 3764 / 3811 and 1965 / 2049; just above the limit, 66^3,
 // 1124 blocks, the pipelined pass is still ahead: 1410 / 1268 and 703 / 697).
-constexpr int kPipeBlocks = 1024;
-
 template <class R>
 bool takes_rows(const Launch<R>& L) {
-  return L.tile == kTileBySize && L.slds && L.nblk <= kRowsBlocks<R>;
+  return !L.plain && L.slds && L.nblk <= kRowsBlocks<R>;
 }
 template <class R>
 bool takes_pipe(const Launch<R>& L) {
-  return L.tile == kTileBySize && L.lds && L.nblk <= kPipeBlocks;
+  return !L.plain && L.lds && L.nblk <= kPipeBlocks;
 }
 
 template <class R>
@@ -3779,7 +3777,7 @@ int launch_flux_ext(int stage, int mode, const Launch<R>& L, int cur, double* rh
     };
     if (L.tile == 2) go(std::integral_constant<int, 2>());
     else if (L.tile == 8) go(std::integral_constant<int, 8>());
-    else go(std::integral_constant<int, kTileBySize>());
+    else go(std::integral_constant<int, kTile>());
     return check();
   }
   if (mode == 0) hipLaunchKernelGGL((k_flux<R, 1, 0>), grid, block, 0, s, L.I, L.bmap, cur, rhs_out);

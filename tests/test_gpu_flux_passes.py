@@ -61,6 +61,17 @@ for dims, prec, tile in json.loads(sys.argv[1]):
     solver = kernels(lambda: s.advance_solution(1))
     s.close()
     out.append([batch, solver])
+# tuned while large, then shrunk
+for prec in (0, 1):
+    p = parse_params(tgv_params(sgs="NONE") + "PRECISION " + ("MIXED" if prec else "FP64") + "\\n")
+    b = Batch(prec)
+    b.set_option("graph", 0)
+    ids = [b.add(m, p, *m.ic_tgv(0.1, 1.4)) for m in (Mesh.lattice((65, 64, 64)), Mesh.lattice(12))]
+    b.tune(2)
+    b.remove(ids[0])
+    b.step(1)
+    out.append([kernels(lambda: b.step(1)), b.tune(2).splitlines()[-1], b.tune(2).splitlines()[-1]])
+    b.close()
 print("TRACE " + json.dumps(out))
 """
 
@@ -87,6 +98,16 @@ def traces():
     assert r.returncode == 0, r.stderr[-2000:]
     line = [x for x in r.stdout.splitlines() if x.startswith("TRACE ")][-1]
     return json.loads(line[6:])
+
+
+# a batch tuned beyond the pipelined pass, whichever tile was kept there, takes the
+# passes of its size once solves have left; those do not read the tile, and the tuner
+# leaves it alone
+@pytest.mark.parametrize("prec", [0, 1])
+def test_tuned_batch_that_shrinks(traces, prec):
+    names, again, once_more = traces[len(ROUTES) + prec]
+    assert [n.split("<")[0] for n in names if n.startswith("k_flux")] == [R] * 3, names
+    assert again.split("tile")[1] == once_more.split("tile")[1]
 
 
 def route_id(i):
